@@ -31,6 +31,7 @@
 #include "abi_common.hpp"
 #include "gemm_common.hpp"
 #include "nf4_device.hpp"
+#include "nf4_skinny.hpp"
 
 namespace nf4s {
 
@@ -1705,6 +1706,20 @@ static int32_t gemm_fwd_groups(const uint16_t *x, const nf4s_tensor *ws, const i
   if (rc == NF4S_OK) rc = check_offsets(k);
   if (rc != NF4S_OK) return rc;
   if (m == 0) return NF4S_OK;
+  if (skinny_takes(ns, count, m)) {
+    SkinnyArgs a{};
+    a.x = x;
+    a.m = m;
+    a.k = k;
+    a.ngroups = count;
+    for (int32_t i = 0; i < count; ++i) {
+      a.grp[i].packed = ws[i].packed;
+      a.grp[i].am = absmax_of(ws[i]);
+      a.grp[i].out = ys[i];
+      a.grp[i].n = ns[i];
+    }
+    return skinny_fwd(a, s, work, work_bytes);
+  }
   // Kind of each weight: bit 0 double-quant, bit 1 batched loads.
   int kind[kMaxGroups];
   for (int32_t i = 0; i < count; ++i)
@@ -1759,6 +1774,21 @@ static int32_t gemm_swiglu(const uint16_t *x, const nf4s_tensor *wg, const nf4s_
     return fail(NF4S_ERR_UNSUPPORTED_SHAPE,
                 "gate and up weights must both be double-quantized or both not");
   if (m == 0) return NF4S_OK;
+  if (skinny_takes(&ff, 1, m)) {
+    SkinnyArgs a{};
+    a.x = x;
+    a.m = m;
+    a.k = k;
+    a.ngroups = 2;
+    const nf4s_tensor *w[2] = {wg, wu};
+    for (int i = 0; i < 2; ++i) {
+      a.grp[i].packed = w[i]->packed;
+      a.grp[i].am = absmax_of(*w[i]);
+      a.grp[i].out = hidden;
+      a.grp[i].n = ff;
+    }
+    return skinny_swiglu(a, s);
+  }
   GroupedArgs ga{};
   GemmArgs &g = ga.base;
   g.a = x;
@@ -1859,6 +1889,7 @@ static int64_t fwd_workspace_bytes(const int64_t *ns, int32_t count, int64_t m, 
   if (m <= 0 || m > kMaxDim || k <= 0 || k > kMaxDim || k % 64 != 0) return 0;
   for (int32_t i = 0; i < count; ++i)
     if (ns[i] <= 0 || ns[i] > kMaxDim) return 0;
+  if (skinny_takes(ns, count, m)) return skinny_workspace_bytes(ns, count, m, k);
   const int64_t tiles_m = (m + kTileM - 1) / kTileM;
   int64_t best = 0;
   for (uint32_t set = 1; set < (1u << count); ++set) {
