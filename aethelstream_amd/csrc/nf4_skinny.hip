@@ -1,4 +1,4 @@
-// nf4_skinny.hip - NF4-dequant-fused forward GEMM for few tokens (m <= 64)
+// nf4_skinny.hip - NF4-dequant-fused forward GEMM for few tokens (m <= 128)
 // on gfx950: y[m,n] = x[m,k] . W^T, and its SwiGLU form.
 //
 // With few tokens the product is bound by reading W (0.52 B per element) and
@@ -181,11 +181,11 @@ __device__ __forceinline__ bool sk_vec_ok(const uint16_t *out, int64_t ldo) {
   return ((reinterpret_cast<uintptr_t>(out) & 7) == 0) && ((ldo & 3) == 0);
 }
 
-// TR: token rows in LDS (4, 16, 32, 64 >= m).  SwiGLU: even waves of a
+// TR: token rows in LDS (4, 16, 32, 64, 128 >= m).  SwiGLU: even waves of a
 // k-group take 32 gate rows, odd ones the same 32 up rows, and hidden is
 // elementwise between their partial tiles.
 template <int TR, int WN, int WK, bool kSwiglu, bool kDQ>
-__global__ void __launch_bounds__(64 * WN * WK, 4) nf4_skinny_kernel(const SkinnyArgs a) {
+__global__ void __launch_bounds__(64 * WN * WK, TR < 128 ? 4 : 2) nf4_skinny_kernel(const SkinnyArgs a) {
   static_assert(!kSwiglu || WN % 2 == 0, "gate and up rows in pairs of waves");
   constexpr int TM = TR < 32 ? 1 : TR / 32;
   constexpr int kCols = 32 * (kSwiglu ? WN / 2 : WN);  // output columns of the workgroup
@@ -390,15 +390,19 @@ __global__ void __launch_bounds__(256) nf4_skinny_sum_kernel(const SkinnyArgs a,
   sk_store4(out + tok * n, col, n, sk_vec_ok(out, n), o);
 }
 
-// The workgroup shape for m tokens: 64 KB of LDS or less, two workgroups a CU.
+// The workgroup shape for m tokens: up to 64 tokens 64 KB of LDS or less, two
+// workgroups a CU.
 // As few weight rows as the x traffic allows (each 32-row block re-reads x
 // from L2), so that the K split stays inside the workgroup.  Measured against
 // it, 28672 x 8192 and 4096 x 4096: four-wave workgroups for m <= 16, 44.9
 // and 9.9 us (43.4 and 8.6); {32, 4, 4} for m = 32, 55.2 and 17.1 (54.9 and
 // 13.2); {64, 4, 4} for m = 64, 78.3 and 22.5 (68.6 and 15.9).
-// Beyond 64 tokens every x fragment still feeds only one MFMA per wave, and
-// the LDS reads of all waves take as long as the MFMAs: the tiled kernel of
-// nf4_gemm.hip, whose waves share the dequantized weights instead, takes over.
+// Up to 128 tokens, 128 KB: every x fragment still feeds only one MFMA per
+// wave, so the LDS reads of all waves take as long as the MFMAs, but at 100
+// tokens it beats the tiled kernel's 128-row tiles (28672 x 8192 88 us against
+// 96, 4096 x 4096 21 against 25; 512-row tiles took 175 and 42).  Beyond them
+// the wave has no registers for more tokens: the tiled kernel, whose waves
+// share the dequantized weights instead, takes over.
 struct SkShape {
   int tr, wn, wk;
 };
@@ -406,14 +410,15 @@ static SkShape sk_shape(int64_t m, bool swiglu) {
   if (m <= 4 && !swiglu) return {4, 1, 8};
   if (m <= 16) return swiglu ? SkShape{16, 2, 4} : SkShape{16, 1, 8};
   if (m <= 32) return {32, 2, 4};
-  return {64, 4, 2};
+  if (m <= 64) return {64, 4, 2};
+  return {128, 4, 2};
 }
 
 // K slices of a launch of `tiles` output tiles: as many as two workgroups a
 // CU take at once, each wave keeping at least 4 steps (fewer would spend more
 // on the partials than on the weights).
 static int sk_slices(int64_t tiles, int64_t steps, const SkShape &sh) {
-  const int64_t slots = 2 * (int64_t)cu_slots();  // 64 KB of LDS each
+  const int64_t slots = (sh.tr == 128 ? 1 : 2) * (int64_t)cu_slots();  // 128 or 64 KB of LDS
   int64_t s = slots / tiles;
   const int64_t most = steps / (4 * sh.wk);  // at least 4 steps per wave
   if (s > most) s = most;
@@ -455,7 +460,8 @@ static void sk_launch(const SkinnyArgs &a, const SkShape &sh, uint32_t grid, hip
         hipLaunchKernelGGL((nf4_skinny_kernel<16, 1, 8, false, kDQ>), g, b, 0, s, a);
       break;
     case 32: hipLaunchKernelGGL((nf4_skinny_kernel<32, 2, 4, kSwiglu, kDQ>), g, b, 0, s, a); break;
-    default: hipLaunchKernelGGL((nf4_skinny_kernel<64, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
+    case 64: hipLaunchKernelGGL((nf4_skinny_kernel<64, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
+    default: hipLaunchKernelGGL((nf4_skinny_kernel<128, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
   }
 }
 

@@ -8,7 +8,7 @@
 namespace nf4s {
 
 // Largest token count the few-token forward takes.
-constexpr int64_t kSkinnyMaxM = 64;
+constexpr int64_t kSkinnyMaxM = 128;
 
 constexpr int kSkinnyMaxGroups = 4;
 

@@ -166,7 +166,7 @@ int32_t nf4s_dequant_batch_bf16(const nf4s_tensor *ts, const int64_t *ns,
  * Requires k % 64 == 0, block_size 64 << s (64 as the reference writes,
  * or 128, 256, ...; shard_engine/src/index.rs:33 lets the index name any)
  * with k % block_size == 0, x/y 16-byte aligned.  Block sizes above 64 run
- * the per-step weight loads (64 takes the batched ones).  Up to 64 tokens
+ * the per-step weight loads (64 takes the batched ones).  Up to 128 tokens
  * run a kernel of their own (each weight dequantized once, in the registers
  * of the lane that multiplies it).  Every GEMM
  * entry point takes m, n and k up to 2^39 (tile counts are 32-bit; the launch
@@ -262,7 +262,7 @@ int32_t nf4s_gemm_dgrad_workspace_size(const int64_t *ns, int32_t count,
  * workspace may be NULL or smaller than nf4s_gemm_fwd_workspace_size
  * reports: the call then runs without the split.  Calls that share a
  * workspace must not overlap (one stream, or ordered streams).  With up to
- * 64 tokens the workspace holds [slice][token][column] partials instead.
+ * 128 tokens the workspace holds [slice][token][column] partials instead.
  */
 int32_t nf4s_gemm_fwd_grouped_ws(const uint16_t *x, const nf4s_tensor *ws,
                                  const int64_t *ns, uint16_t *const *ys,

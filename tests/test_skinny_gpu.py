@@ -1,5 +1,5 @@
-"""The few-token forward (m <= 64) against an fp64 product over the bf16
-dequantized weights, at the edges of its token tiles (4, 16, 32, 64 rows),
+"""The few-token forward (m <= 128) against an fp64 product over the bf16
+dequantized weights, at the edges of its token tiles (4, 16, 32, 64, 128 rows),
 weight tiles (32 rows) and reduction steps (128 deep, k % 128 == 64 leaving
 half a step; fewer steps than k-groups), for both absmax forms and block
 sizes, grouped, SwiGLU, split over K slices or not, and unaligned outputs.
@@ -41,7 +41,7 @@ def _close(y, ref):
     assert err <= TOL, err
 
 
-@pytest.mark.parametrize("m", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 128])
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129])
 @pytest.mark.parametrize("n,k", [(1, 64), (31, 192), (96, 128), (130, 1088), (4096, 4096)])
 @pytest.mark.parametrize("dq", [False, True])
 def test_fwd_tile_edges(m, n, k, dq):
@@ -52,7 +52,7 @@ def test_fwd_tile_edges(m, n, k, dq):
     _close(gemm.linear_fwd(x, w, split_k=False), ref)
 
 
-@pytest.mark.parametrize("m", [1, 16, 20, 60])
+@pytest.mark.parametrize("m", [1, 16, 20, 60, 100])
 @pytest.mark.parametrize("block", [64, 128, 256])
 def test_grouped_kinds_and_blocks(m, block):
     k = 2816 if block != 256 else 2816 // 256 * 256
@@ -65,7 +65,7 @@ def test_grouped_kinds_and_blocks(m, block):
             _close(y, _ref(x, w))
 
 
-@pytest.mark.parametrize("m", [1, 16, 17, 64, 77])
+@pytest.mark.parametrize("m", [1, 16, 17, 64, 77, 128])
 @pytest.mark.parametrize("ff,k", [(5, 64), (192, 320), (1000, 4096)])
 @pytest.mark.parametrize("dq", [False, True])
 def test_swiglu(m, ff, k, dq):
@@ -75,7 +75,7 @@ def test_swiglu(m, ff, k, dq):
     _close(gemm.linear_swiglu(x, wg, wu), gate * torch.sigmoid(gate) * _ref(x, wu))
 
 
-@pytest.mark.parametrize("m", [3, 24, 48])
+@pytest.mark.parametrize("m", [3, 24, 48, 128])
 @pytest.mark.parametrize("dq", [False, True])
 def test_one_hot_equals_dequantized_weight(m, dq):
     # 1.0 * W[n, j] added onto exact zeros: every output is a weight, bit for bit.
