@@ -63,7 +63,9 @@ __device__ __forceinline__ float load_elem<uint16_t>(const uint16_t *x, int64_t 
   return __builtin_bit_cast(float, (uint32_t)x[e] << 16);
 }
 
-// ---- Block-64 quantize: 8 elements per lane, 8 lanes per block ----------
+// ---- Power-of-two blocks: 8 elements per lane, 2^kLanes lanes per block ----
+// (kLanes = 3 for the 64-element blocks the writer produces; 8 to 512
+// elements, kLanes = 0 to 6, for the others the shard index allows.)
 //
 // The code rule above is monotone in n (within a bracket the rounded
 // distance to the lower code only grows and to the upper one only shrinks),
@@ -169,23 +171,41 @@ __device__ __forceinline__ uint32_t dpp_umax(uint32_t m) {
   return (o > m) ? o : m;
 }
 
+// Unsigned max over the aligned group of 2^kLanes lanes, in each of them: quad
+// xor 1, quad xor 2, half-row mirror and row mirror by DPP, then the row pairs
+// and the wave's halves by permlane swaps.
+template <int kLanes>
+__device__ __forceinline__ uint32_t lanes_umax(uint32_t m) {
+  if constexpr (kLanes > 0) m = dpp_umax<0xB1>(m);   // quad_perm [1,0,3,2]
+  if constexpr (kLanes > 1) m = dpp_umax<0x4E>(m);   // quad_perm [2,3,0,1]
+  if constexpr (kLanes > 2) m = dpp_umax<0x141>(m);  // row_half_mirror: i <-> 7-i within 8
+  if constexpr (kLanes > 3) m = dpp_umax<0x140>(m);  // row_mirror: i <-> 15-i within 16
+  if constexpr (kLanes > 4) {
+    const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    const uint32_t a = r[0], b = r[1];
+    m = (a > b) ? a : b;
+  }
+  if constexpr (kLanes > 5) {
+    const auto r = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    const uint32_t a = r[0], b = r[1];
+    m = (a > b) ? a : b;
+  }
+  return m;
+}
+
 // Codes of the lane's 8 elements, packed as quantizer.py:43-46 packs them
 // (even element in the high nibble), and the block's unclamped absmax
 // (:35, :48-53) in every lane of the block.  Call with the whole wave
-// active: the absmax is reduced across the block's 8 lanes with DPP moves
-// (quad xor 1, quad xor 2, half-row mirror) on the bit patterns of |x|,
-// whose unsigned order is the numeric order with NaN above +inf (torch's
-// max propagates NaN).
-template <bool kFull>
+// active: the absmax is reduced across the block's lanes on the bit patterns
+// of |x|, whose unsigned order is the numeric order with NaN above +inf
+// (torch's max propagates NaN).
+template <bool kFull, int kLanes>
 __device__ __forceinline__ float encode8(const uint2 *tab, const float v[8], int64_t e0,
                                          int64_t lim, uint32_t &word) {
   float ml = __builtin_elementwise_maximum(fabsf(v[0]), fabsf(v[1]));  // NaN-propagating
 #pragma unroll
   for (int k = 2; k < 8; ++k) ml = __builtin_elementwise_maximum(ml, fabsf(v[k]));
-  uint32_t mb = __builtin_bit_cast(uint32_t, ml);
-  mb = dpp_umax<0xB1>(mb);   // quad_perm [1,0,3,2]
-  mb = dpp_umax<0x4E>(mb);   // quad_perm [2,3,0,1]
-  mb = dpp_umax<0x141>(mb);  // row_half_mirror: lane i <-> 7-i within 8
+  const uint32_t mb = lanes_umax<kLanes>(__builtin_bit_cast(uint32_t, ml));
   const float m = __builtin_bit_cast(float, mb);
   uint32_t c[8];
   // NaN, inf and absmax >= 2^126 (rcp would be subnormal) take the exact path.
@@ -210,14 +230,14 @@ __device__ __forceinline__ float encode8(const uint2 *tab, const float v[8], int
   return m;
 }
 
-// A tile is 8 blocks (512 elements) by one wave; lane l holds elements
+// A tile is 512 elements (512 / block size blocks) by one wave; lane l holds elements
 // 8l .. 8l+7 of it, so the wave reads 2 KB (fp32) and writes 256 B
 // contiguously.  tile_e0(t) is the first element of tile t and
 // absmax_out(t, j, m) takes block j of tile t.
 
 // One tile with every access guarded: elements at or past `lim` read as
 // absent and are not written (the last, partial tile; unaligned buffers).
-template <typename T, typename AbsmaxOut>
+template <typename T, int kLanes, typename AbsmaxOut>
 __device__ __forceinline__ void quantize_tile_guarded(const T *__restrict__ x, int64_t lim,
                                                       int64_t t, int64_t tile_e0,
                                                       const uint2 *tab,
@@ -228,23 +248,23 @@ __device__ __forceinline__ void quantize_tile_guarded(const T *__restrict__ x, i
   float v[8];
   load8_guarded<T>(x, lim, e0, v);
   uint32_t word;
-  const float m = encode8<false>(tab, v, e0, lim, word);
+  const float m = encode8<false, kLanes>(tab, v, e0, lim, word);
   if (e0 < lim) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (e0 + 2 * j < lim) packed[(e0 >> 1) + j] = (uint8_t)(word >> (8 * j));
-    if ((lane & 7) == 0) absmax_out(t, lane >> 3, m);
+    if ((lane & ((1 << kLanes) - 1)) == 0) absmax_out(t, lane >> kLanes, m);
   }
 }
 
 // Chunks of kU full tiles (x 16-byte and packed 4-byte aligned): one wave
 // takes chunks c0, c0 + dc, ... < nchunks, with the next chunk's loads
 // issued before the current chunk's codes (two register sets, alternating).
-// Every path through a chunk issues the same loads and stores (all 8 lanes
+// Every path through a chunk issues the same loads and stores (all lanes
 // of a block store its absmax, the same value to the same address; the
 // loop's exits each get their own copy of the codes), so the wait before a
 // chunk's codes leaves the next chunk's loads and the last stores in flight.
-template <typename T, int kU, typename TileE0, typename AbsmaxOut>
+template <typename T, int kU, int kLanes, typename TileE0, typename AbsmaxOut>
 __device__ __forceinline__ void quantize_wave_full(const T *__restrict__ x, int64_t nchunks,
                                                    int64_t c0, int64_t dc, const uint2 *tab,
                                                    uint8_t *__restrict__ packed, TileE0 tile_e0,
@@ -262,9 +282,9 @@ __device__ __forceinline__ void quantize_wave_full(const T *__restrict__ x, int6
       const int64_t t = c * kU + u;
       const int64_t e0 = tile_e0(t) + 8 * lane;
       uint32_t word;
-      const float m = encode8<true>(tab, v[u], e0, 0, word);
+      const float m = encode8<true, kLanes>(tab, v[u], e0, 0, word);
       *(uint32_t *)(packed + (e0 >> 1)) = word;
-      absmax_out(t, lane >> 3, m);
+      absmax_out(t, lane >> kLanes, m);
     }
   };
   load(va, c0);
@@ -291,7 +311,7 @@ __device__ __forceinline__ void quantize_wave_full(const T *__restrict__ x, int6
 // of `nw`: whole chunks of full tiles through the pipelined path when kVec,
 // the rest (the partial last tile, full tiles short of a chunk, every tile
 // when !kVec) guarded.
-template <typename T, bool kVec, int kU, typename TileE0, typename AbsmaxOut>
+template <typename T, bool kVec, int kU, int kLanes, typename TileE0, typename AbsmaxOut>
 __device__ __forceinline__ void quantize_range(const T *__restrict__ x, int64_t lim,
                                                int64_t ntiles, int64_t wid, int64_t nw,
                                                const uint2 *tab, uint8_t *__restrict__ packed,
@@ -300,30 +320,33 @@ __device__ __forceinline__ void quantize_range(const T *__restrict__ x, int64_t 
   if (kVec) {
     const int64_t nfull = (tile_e0(ntiles - 1) + 512 <= lim) ? ntiles : ntiles - 1;
     const int64_t nchunks = nfull / kU;
-    quantize_wave_full<T, kU>(x, nchunks, wid, nw, tab, packed, tile_e0, absmax_out);
+    quantize_wave_full<T, kU, kLanes>(x, nchunks, wid, nw, tab, packed, tile_e0, absmax_out);
     t0 = nchunks * kU;
   }
   for (int64_t t = t0 + wid; t < ntiles; t += nw)
-    quantize_tile_guarded<T>(x, lim, t, tile_e0(t), tab, packed, absmax_out);
+    quantize_tile_guarded<T, kLanes>(x, lim, t, tile_e0(t), tab, packed, absmax_out);
 }
 
 // kVec: x 16-byte and packed 4-byte aligned (16-byte loads, 4-byte stores).
-template <typename T, bool kVec, int kU>
-__global__ void __launch_bounds__(256) quantize64_kernel(const T *__restrict__ x, int64_t n,
+// Blocks of 8 << kLanes elements.
+template <typename T, bool kVec, int kU, int kLanes>
+__global__ void __launch_bounds__(256) quantize_kernel(const T *__restrict__ x, int64_t n,
                                                          uint8_t *__restrict__ packed,
                                                          float *__restrict__ absmax,
                                                          int64_t ntiles) {
   __shared__ uint2 tab[kStepTableWords];
   init_step_table(tab);
   __syncthreads();
-  quantize_range<T, kVec, kU>(
+  quantize_range<T, kVec, kU, kLanes>(
       x, n, ntiles, (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
       (int64_t)gridDim.x * 4, tab,
       packed, [](int64_t t) { return t * 512; },
-      [=](int64_t t, int j, float m) { absmax[t * 8 + j] = m; });  // :48-53, unclamped
+      [=](int64_t t, int j, float m) {
+        absmax[t * (64 >> kLanes) + j] = m;  // :48-53, unclamped
+      });
 }
 
-// Any block size: per-block absmax, then per-byte codes.
+// Any other block size: per-block absmax, then per-byte codes.
 __global__ void absmax_generic_kernel(const float *__restrict__ x, int64_t n, int32_t bs,
                                       float *__restrict__ absmax, int64_t nblocks) {
   for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < nblocks;
@@ -403,9 +426,9 @@ __global__ void __launch_bounds__(256) dq_encode_kernel(const float *__restrict_
 // after apply_galore_bf16_update, doublepass/src/precision.rs:187-202): each
 // workgroup takes groups of `group` 64-element blocks in turn (a grid of at
 // most kQuantMaxGrid), its waves taking a group's 8-block tiles in turn (the
-// same lane code as quantize64_kernel).
+// same lane code as quantize_kernel).
 // The block absmax stay in LDS (never written as fp32), so the call needs no
-// scratch memory; codes come from the fp32 absmax exactly as quantize64_kernel
+// scratch memory; codes come from the fp32 absmax exactly as quantize_kernel
 // computes them, and q / scale exactly as dq_encode_kernel does.
 template <typename T, bool kVec, int kU>
 __global__ void __launch_bounds__(256) quantize_dq_kernel(const T *__restrict__ x, int64_t n,
@@ -427,7 +450,7 @@ __global__ void __launch_bounds__(256) quantize_dq_kernel(const T *__restrict__ 
     // Elements of this group's blocks: the others read as absent, so a tile
     // that runs past the group (group < 8) neither counts nor writes them.
     const int64_t lim = (64 * (b0 + nb) < n) ? 64 * (b0 + nb) : n;
-    quantize_range<T, kVec, kU>(
+    quantize_range<T, kVec, kU, 3>(
         x, lim, (nb + 7) >> 3, __builtin_amdgcn_readfirstlane(wave), 4, tab, packed,
         [=](int64_t t) { return (b0 + 8 * t) * 64; },
         [=](int64_t t, int j, float m) { am_lds[8 * t + j] = m; });
@@ -630,25 +653,26 @@ static int32_t dequant_batch(const nf4s_tensor *ts, const int64_t *ns, uint16_t 
 }
 
 constexpr int kQuantU = 1;         // tiles per chunk
-constexpr int kQuantMaxGrid = 1024;  // workgroups of the block-64 quantize launches
+constexpr int kQuantMaxGrid = 1024;  // workgroups of the quantize launches
 
 template <typename T>
 static bool quantize_vec_ok(const T *x, const uint8_t *packed) {
   return ((uintptr_t)x % 16 == 0) && ((uintptr_t)packed % 4 == 0);
 }
 
-template <typename T>
-static int32_t quantize64(const T *x, int64_t n, uint8_t *packed, float *absmax, hipStream_t s) {
+template <typename T, int kLanes>
+static int32_t quantize_lanes(const T *x, int64_t n, uint8_t *packed, float *absmax,
+                              hipStream_t s) {
   const int64_t ntiles = ceil_div(n, 512);
   int64_t grid = ((ntiles + kQuantU - 1) / kQuantU + 3) / 4;
   if (grid > kQuantMaxGrid) grid = kQuantMaxGrid;
   if (quantize_vec_ok(x, packed))
-    hipLaunchKernelGGL((quantize64_kernel<T, true, kQuantU>), dim3((uint32_t)grid), dim3(256), 0, s, x, n,
-                       packed, absmax, ntiles);
+    hipLaunchKernelGGL((quantize_kernel<T, true, kQuantU, kLanes>), dim3((uint32_t)grid),
+                       dim3(256), 0, s, x, n, packed, absmax, ntiles);
   else
-    hipLaunchKernelGGL((quantize64_kernel<T, false, kQuantU>), dim3((uint32_t)grid), dim3(256), 0, s, x, n,
-                       packed, absmax, ntiles);
-  return check_launch("quantize64_kernel");
+    hipLaunchKernelGGL((quantize_kernel<T, false, kQuantU, kLanes>), dim3((uint32_t)grid),
+                       dim3(256), 0, s, x, n, packed, absmax, ntiles);
+  return check_launch("quantize_kernel");
 }
 
 template <typename T>
@@ -694,7 +718,19 @@ int32_t nf4s_quantize(const float *x, int64_t n, int32_t block_size, uint8_t *pa
     return fail(NF4S_ERR_INVALID_ARGUMENT, "NULL buffer");
   const int64_t nb = ceil_div(n, block_size);
   hipStream_t s = as_stream(stream);
-  if (block_size == 64) return quantize64<float>(x, n, packed, absmax, s);
+  // Powers of two from 8 to 512: a block within one wave's tile, one pass over
+  // x.  fp32 4099 x 4096 in blocks of 128: 104.1 -> 12.7 us against the two
+  // kernels below, which read x twice, 512 bytes apart between lanes.
+  switch (block_size) {
+    case 8: return quantize_lanes<float, 0>(x, n, packed, absmax, s);
+    case 16: return quantize_lanes<float, 1>(x, n, packed, absmax, s);
+    case 32: return quantize_lanes<float, 2>(x, n, packed, absmax, s);
+    case 64: return quantize_lanes<float, 3>(x, n, packed, absmax, s);
+    case 128: return quantize_lanes<float, 4>(x, n, packed, absmax, s);
+    case 256: return quantize_lanes<float, 5>(x, n, packed, absmax, s);
+    case 512: return quantize_lanes<float, 6>(x, n, packed, absmax, s);
+    default: break;
+  }
   hipLaunchKernelGGL(absmax_generic_kernel, dim3(grid_for(nb, 256)), dim3(256), 0, s, x, n,
                      block_size, absmax, nb);
   int32_t rc = check_launch("absmax_generic_kernel");
@@ -715,7 +751,7 @@ int32_t nf4s_quantize_bf16(const uint16_t *x, int64_t n, int32_t block_size, uin
   if (n == 0) return NF4S_OK;
   if (x == nullptr || packed == nullptr || absmax == nullptr)
     return fail(NF4S_ERR_INVALID_ARGUMENT, "NULL buffer");
-  return quantize64<uint16_t>(x, n, packed, absmax, as_stream(stream));
+  return quantize_lanes<uint16_t, 3>(x, n, packed, absmax, as_stream(stream));
 }
 
 int32_t nf4s_quantize_dq(const float *x, int64_t n, int32_t block_size, int32_t group,
