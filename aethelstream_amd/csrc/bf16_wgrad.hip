@@ -41,7 +41,6 @@ struct WgradArgs {
   const uint16_t *x;  // [M, K], row stride K
   int64_t M, K;
   int32_t tiles_n, tiles_k;
-  int32_t accumulate;
   int32_t blk_n, blk_k;  // XCD block of blk_n x blk_k tiles (0: map_tile order)
 };
 
@@ -205,7 +204,117 @@ __device__ __forceinline__ void wgrad_close_step(int64_t t, int64_t nsteps) {
   });
 }
 
+// Direct epilogue, for ragged columns and outputs without 16-byte stores: four
+// adjacent fp32 per store.
+template <bool kAcc>
+__device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[4][4], float *dw,
+                                         int64_t n0, int64_t k0, int64_t N, int lane,
+                                         bool vec_ok) {
+  asm volatile("" : "+v"(lane));  // as in wg_store_lds
+  const int jl = lane & 31, grp = lane >> 5;
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    const int64_t n = n0 + 32 * mt + jl;
+    if (n < N) {
+      float *row = dw + n * g.K;
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int64_t k = k0 + 32 * nt + 8 * j + 4 * grp;
+          floatx4 v = {acc[mt][nt][4 * j], acc[mt][nt][4 * j + 1], acc[mt][nt][4 * j + 2],
+                       acc[mt][nt][4 * j + 3]};
+          if (vec_ok && k + 4 <= g.K) {
+            floatx4 *p = reinterpret_cast<floatx4 *>(row + k);
+            if constexpr (kAcc) v += *p;
+            *p = v;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (k + i < g.K) row[k + i] = kAcc ? row[k + i] + v[i] : v[i];
+          }
+        }
+    }
+  }
+}
+
+// Epilogue through LDS for whole-width tiles: the direct stores write 32 rows
+// x 32 bytes per instruction, these two whole 512-byte rows.  Per 32-row block
+// mt the wave writes its 32 x 128 fp32 to its own 16 KB of the idle ring (row
+// r, 16-byte chunk c at physical chunk c ^ r: the lanes of a ds_write_b128
+// share c, those of a ds_read_b128 r, both spread over all banks), reads it
+// back by rows and stores; to accumulate, 8 of dW's old row pairs are loaded
+// at a time.  The tile's output burst (64 MB a round over the chip) is what a
+// short reduction waits for: against the direct stores, same box, 2 x 11008 x
+// 4096 over 1000 tokens 245 -> 231 us (326 -> 273 accumulating), 28672 x 8192
+// over 512 tokens 384 -> 319 (600 -> 484), 8192 x 8192 over 8192 tokens 846 ->
+// 826 (909 -> 867).  Non-temporal stores: without them 367 us for 28672 x 8192
+// over 512 tokens.  Accumulating is its own instantiation: as a run-time test
+// it spilled 51 registers in both.
+template <bool kAcc>
+__device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 (&acc)[4][4],
+                                             floatx4 *lds, float *dw, int64_t n0, int64_t k0,
+                                             int64_t N, int lane) {
+  // An opaque lane index keeps the per-lane addresses below from being hoisted
+  // out of the tile loop and spilled.
+  asm volatile("" : "+v"(lane));
+  const int jl = lane & 31, grp = lane >> 5;
+  const int r0 = lane >> 5, c = lane & 31;  // read-back: row 2i + r0, chunk c
+  // The wave's rows below N through a buffer resource that ends after the last.
+  const int64_t left = N - n0;
+  const int64_t rows = left <= 0 ? 0 : (left > 128 ? 128 : left);
+  const uint32_t ld4 = (uint32_t)(g.K * 4);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(rows > 0 ? dw + n0 * g.K + k0 : dw), 0,
+      rows > 0 ? (int32_t)((rows - 1) * ld4 + 512) : 0, kBufferFlags);
+  typedef unsigned int uvec4 __attribute__((ext_vector_type(4)));
+  constexpr int kStoreNt = 2;  // non-temporal
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    const uint32_t base = (uint32_t)(32 * mt + r0) * ld4 + 16u * (uint32_t)c;
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        lds[jl * 32 + ((8 * nt + 2 * j + grp) ^ jl)] =
+            (floatx4){acc[mt][nt][4 * j], acc[mt][nt][4 * j + 1], acc[mt][nt][4 * j + 2],
+                      acc[mt][nt][4 * j + 3]};
+    // Other lanes' writes are read below, and the reads end before the next
+    // block's writes.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < 16; h += 8) {
+      floatx4 v[8], old[8];
+      if constexpr (kAcc) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          old[i] = __builtin_bit_cast(
+              floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                           rs, (int)(base + 2u * (uint32_t)(h + i) * ld4), 0, 0));
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 2 * (h + i) + r0;
+        v[i] = lds[r * 32 + (c ^ r)];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (kAcc) v[i] += old[i];
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(uvec4, v[i]), rs,
+            (int)(base + 2u * (uint32_t)(h + i) * ld4), 0, kStoreNt);
+      }
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+    asm volatile("" ::: "memory");
+  }
+}
+
 // One output tile: its 256 x 256 dW block over all M tokens.
+template <bool kAcc>
 __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g) {
   const int T = g.tiles_n * g.tiles_k;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -223,6 +332,8 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
     ldy[i] = reinterpret_cast<char *>(&g_wg_lds[i][0][0]);
     lx[i] = reinterpret_cast<char *>(&g_wg_lds[i][1][0]);
   }
+  // 16 KB of the ring for each wave's epilogue.
+  floatx4 *lds_wave = reinterpret_cast<floatx4 *>(&g_wg_lds[0][0][0]) + 1024 * wave;
   const int64_t nsteps = (g.M + kWgStep - 1) / kWgStep;
   const uint32_t step_x = (uint32_t)(kWgStep * g.K * 2);
 #pragma unroll 1
@@ -323,36 +434,15 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
 
     // Epilogue.  Lane l holds dW row n = n0 + 128 hn + 32 mt + l % 32 and
     // columns k = k0 + 128 hk + 32 nt + 8 j + 4 (l / 32) + i in registers
-    // 4 j + i of tile [mt][nt]: four adjacent fp32 per 16-B store.
-    const int jl = lane & 31, grp = lane >> 5;
+    // 4 j + i of tile [mt][nt].
     const bool vec_ok = ((reinterpret_cast<uintptr_t>(dw) & 15) == 0) && ((g.K & 3) == 0);
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      const int64_t n = n0 + 128 * hn + 32 * mt + jl;
-      if (n < N) {
-        float *row = dw + n * g.K;
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int64_t k = k0 + 128 * hk + 32 * nt + 8 * j + 4 * grp;
-            floatx4 v = {acc[mt][nt][4 * j], acc[mt][nt][4 * j + 1], acc[mt][nt][4 * j + 2],
-                         acc[mt][nt][4 * j + 3]};
-            if (vec_ok && k + 4 <= g.K) {
-              floatx4 *p = reinterpret_cast<floatx4 *>(row + k);
-              if (g.accumulate) v += *p;
-              *p = v;
-            } else {
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (k + i < g.K) row[k + i] = g.accumulate ? row[k + i] + v[i] : v[i];
-            }
-          }
-      }
-    }
-    // The next tile's prologue DMAs overwrite stage 0, which the last
-    // step's reads may have used: every wave's reads end before this.
-    step_barrier<0>();
+    if (vec_ok && k0 + kWgTile <= g.K && g.K < ((int64_t)1 << 22))  // 32-bit row offsets
+      wg_store_lds<kAcc>(g, acc, lds_wave, dw, n0 + 128 * hn, k0 + 128 * hk, N, lane);
+    else
+      wg_store<kAcc>(g, acc, dw, n0 + 128 * hn, k0 + 128 * hk, N, lane, vec_ok);
+    // The next tile's prologue DMAs overwrite the LDS that the last step and
+    // the epilogues read: every wave's reads (not its stores) end before this.
+    step_barrier<63>();
   }
 }
 
@@ -398,7 +488,6 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
   g.M = m;
   g.K = k;
   g.tiles_k = (int32_t)((k + kWgTile - 1) / kWgTile);
-  g.accumulate = accumulate ? 1 : 0;
   int64_t tiles_n = 0;
   for (int i = 0; i < count; ++i) {
     const int64_t n = ns[i];
@@ -467,7 +556,10 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
       }
     }
   }
-  hipLaunchKernelGGL(wgrad_kernel, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
+  if (accumulate)
+    hipLaunchKernelGGL(wgrad_kernel<true>, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
+  else
+    hipLaunchKernelGGL(wgrad_kernel<false>, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
   return check_launch("wgrad_kernel");
 }
 
