@@ -31,7 +31,8 @@ from .nf4 import Nf4Weight, _require_cuda, _stream_ptr
 
 
 def _check_act(t: torch.Tensor, cols: int, name: str) -> None:
-    _require_cuda(t)
+    if not (t.is_cuda and t.is_contiguous()):
+        _require_cuda(t)
     if t.dtype != torch.bfloat16:
         raise ValueError(f"{name} must be bfloat16")
     if t.dim() != 2 or t.shape[1] != cols:
@@ -97,11 +98,14 @@ def _workspace_for(need: int, workspace: Optional[torch.Tensor], ref: torch.Tens
     return workspace
 
 
+# Array types of 1 .. 4 elements, built once (index = count).
+_I64S = [ctypes.c_int64 * i for i in range(5)]
+_PTRS = [ctypes.c_void_p * i for i in range(5)]
+_TENSORS = [_lib.Nf4sTensor * i for i in range(5)]
+
+
 def _descs(ws: Sequence[Nf4Weight]):
-    arr = (_lib.Nf4sTensor * len(ws))()
-    for i, w in enumerate(ws):
-        arr[i] = w.descriptor()
-    return arr
+    return _TENSORS[len(ws)](*[w.descriptor() for w in ws])
 
 
 def fwd_workspace_bytes(ns: Sequence[int], m: int, k: int) -> int:
@@ -122,36 +126,41 @@ def linear_fwd_grouped(x: torch.Tensor, ws: Sequence[Nf4Weight],
     share it)."""
     if not 1 <= len(ws) <= 4:
         raise ValueError("linear_fwd_grouped takes 1 to 4 weights")
+    count = len(ws)
     k = int(ws[0].shape[1])
+    widths = [int(w.shape[0]) for w in ws]
     if any(int(w.shape[1]) != k for w in ws):
         raise ValueError("grouped weights must share k")
     _check_act(x, k, "x")
     m = x.shape[0]
-    if outs is None:
-        outs = [torch.empty(m, int(w.shape[0]), dtype=torch.bfloat16, device=x.device)
-                for w in ws]
-    if len(outs) != len(ws):
-        raise ValueError("one output per weight")
-    for w, o in zip(ws, outs):
-        _check_act(o, int(w.shape[0]), "out")
-    ns = (ctypes.c_int64 * len(ws))(*[int(w.shape[0]) for w in ws])
-    ys = (ctypes.c_void_p * len(ws))(*[o.data_ptr() for o in outs])
+    if outs is None:  # bf16, contiguous and [m, n_i] by construction
+        outs = [torch.empty(m, n, dtype=torch.bfloat16, device=x.device) for n in widths]
+    else:
+        if len(outs) != count:
+            raise ValueError("one output per weight")
+        for n, o in zip(widths, outs):
+            _check_act(o, n, "out")
+    ns = _I64S[count](*widths)
+    ys = _PTRS[count](*[o.data_ptr() for o in outs])
     descs = _descs(ws)
-    need = fwd_workspace_bytes(list(ns), m, k) if split_k else 0
+    lib = _lib.load()
+    need = 0
+    if split_k:
+        size = ctypes.c_int64()
+        _lib.check(lib.nf4s_gemm_fwd_workspace_size(ns, count, m, k, ctypes.byref(size)))
+        need = size.value
     if need > 0:
         if workspace is not None and workspace.device != x.device:
             raise ValueError("workspace must be on x's device")
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
         _require_cuda(workspace)
-        if not workspace.is_contiguous():
-            raise ValueError("workspace must be contiguous")
-        _lib.check(_lib.load().nf4s_gemm_fwd_grouped_ws(
-            x.data_ptr(), descs, ns, ys, len(ws), m, k, workspace.data_ptr(),
+        _lib.check(lib.nf4s_gemm_fwd_grouped_ws(
+            x.data_ptr(), descs, ns, ys, count, m, k, workspace.data_ptr(),
             workspace.numel() * workspace.element_size(), _stream_ptr(x)))
     else:
-        _lib.check(_lib.load().nf4s_gemm_fwd_grouped(x.data_ptr(), descs, ns, ys, len(ws), m, k,
-                                                     _stream_ptr(x)))
+        _lib.check(lib.nf4s_gemm_fwd_grouped(x.data_ptr(), descs, ns, ys, count, m, k,
+                                             _stream_ptr(x)))
     return list(outs)
 
 
