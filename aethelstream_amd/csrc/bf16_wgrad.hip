@@ -8,11 +8,13 @@
 // fp32.  The reduction runs over the token index m, the row index of both
 // operands, so both MFMA operands are columns of row-major tiles.
 //
-// Workgroup = 4 waves in 2 x 2, tile = 256 dW rows (n) x 256 dW columns (k);
-// each wave owns 128 x 128 in 256 accumulator registers (16 tiles of
-// v_mfma_f32_32x32x16_bf16).  Per 32-token step the dy tile (32 x 256 bf16)
-// and the x tile (32 x 256) move into LDS with direct-to-LDS loads, into a
-// ring of kWgStages 32 KB stages that keeps the next kWgStages - 1 steps in
+// Workgroup = 4 waves in 2 x 2, tile = 64 kMT dW rows (n) x 256 dW columns (k),
+// kMT = 4 or 2; each wave owns 32 kMT x 128 in 64 kMT accumulator registers
+// (4 kMT tiles of v_mfma_f32_32x32x16_bf16).  kMT = 4 takes a CU for itself,
+// of kMT = 2 two workgroups share one (wg_tile_mt says which is launched).
+// Per 32-token step the dy tile (32 x 64 kMT bf16) and the x tile (32 x 256)
+// move into LDS with direct-to-LDS loads, into a ring of kWgStages stages of
+// 32 (24) KB that keeps the next kWgStages - 1 steps in
 // flight while step t computes (3 stages measured faster than 2 of 64
 // tokens, and than 4 or 5 of 32), and each wave reads its fragments with
 // the transposing ds_read_b64_tr_b16: 8 consecutive tokens of one column
@@ -24,7 +26,7 @@
 namespace nf4s {
 
 constexpr int kWgThreads = 256;
-constexpr int kWgTile = 256;  // dW rows and columns per workgroup
+constexpr int kWgTile = 256;  // dW columns per workgroup
 constexpr int kWgStep = 32;   // tokens per step
 constexpr int kWgStages = 3;  // LDS ring stages
 
@@ -41,7 +43,8 @@ struct WgradArgs {
   const uint16_t *x;  // [M, K], row stride K
   int64_t M, K;
   int32_t tiles_n, tiles_k;
-  int32_t blk_n, blk_k;  // XCD block of blk_n x blk_k tiles (0: map_tile order)
+  int32_t blk_n, blk_k;  // XCD block of blk_n x blk_k tiles (0: strips)
+  int32_t strip;         // tile columns per strip (wg_map_tile)
 };
 
 // a[i] for a wave-uniform i < kMaxWgGroups, as a chain of selects: indexing
@@ -54,17 +57,29 @@ __device__ __forceinline__ T wg_pick(const T (&a)[kMaxWgGroups], int i) {
   return v;
 }
 
-// Tile order of a launch whose rounds are all full (T a multiple of the
-// grid G, G / 8 slots per XCD): in round r, XCD x (workgroups b with
-// b % 8 == x) takes block 8 r + x of blk_n x blk_k tiles, blk_n * blk_k =
-// G / 8, slot i = (b % G) / 8 the tile (i / blk_k, i % blk_k) of the block.
-// The XCD's workgroups then read blk_n dy column blocks and blk_k x column
-// blocks per 64-token step (4 + 8 = 12 x 32 KB on a 256-CU part) instead of
-// 1 + 32 in map_tile's order, where they share one dy block and read every
-// x block of the row; the rest comes from the XCD's L2.
+// Tile order.  An XCD's resident workgroups should form a square-ish patch of
+// the tile grid: they then read few dy and x column blocks per step from
+// memory and the rest from the XCD's L2.
+// A launch whose rounds are all full (T a multiple of the grid G, G / 8 slots
+// per XCD): in round r, XCD x (workgroups b with b % 8 == x) takes block
+// 8 r + x of blk_n x blk_k tiles, blk_n * blk_k = G / 8, slot i = (b % G) / 8
+// the tile (i / blk_k, i % blk_k) of the block.
+// Any other launch: the tiles are numbered row by row within strips of
+// `strip` tile columns (the last one narrower) and each XCD takes a
+// contiguous range of them.  Rows over the whole width instead read every x
+// block for each dy block: 11008 x 16384 over 8192 tokens 2498 us, strips
+// 2295 (256-row tiles); 4096 x 11008 over 4096, 429 and 317 (128-row).
 __device__ __forceinline__ void wg_map_tile(const WgradArgs &g, int b, int &tn, int &tk) {
   if (g.blk_n == 0) {
-    map_tile(b, g.tiles_n, g.tiles_k, tn, tk);
+    const int T = g.tiles_n * g.tiles_k;
+    const int x = b & 7, base = T >> 3, rem = T & 7;
+    const int L = x * base + (x < rem ? x : rem) + (b >> 3);
+    const int per = g.tiles_n * g.strip;  // tiles of a whole strip
+    const int s = L / per, i = L - s * per;
+    const int left = g.tiles_k - s * g.strip;
+    const int w = left < g.strip ? left : g.strip;
+    tn = i / w;
+    tk = s * g.strip + i - tn * w;
     return;
   }
   const int G = gridDim.x;
@@ -76,19 +91,24 @@ __device__ __forceinline__ void wg_map_tile(const WgradArgs &g, int b, int &tn, 
   tk = bk * g.blk_k + i % g.blk_k;
 }
 
-// LDS tile: 32 token rows x 256 columns (512 B = 32 units of 16 B per row).
-// A wave reads one 128-column half (16 units).  Unit u of row r lives at
+// LDS tile: 32 token rows x 256 columns (512 B = 32 units of 16 B per row), or
+// 128 columns (16 units) of dy when kMT = 2.  A wave reads one half of the
+// columns.  Unit u of row r lives at
 // physical unit (u & 16) | ((u & 15) ^ 5 (r % 4)): with it, each 32-lane
 // half of a transposed fragment read covers 16 distinct 16-B units of one
-// half-row's 64 banks (rows are 512 B = 128 banks apart, so every row starts
-// at bank 0), and each 16-lane quarter of a DMA writes one row's 16
+// half-row's 64 banks (rows are 512 B or 256 B = 128 or 64 banks apart, so every
+// row starts at bank 0), and each 16-lane quarter of a DMA writes one row's 16
 // contiguous units.
 __device__ __forceinline__ int wg_unit(int row, int u) {
   return (u & 16) | ((u & 15) ^ (5 * (row & 3)));
 }
 
-// [stage][operand 0 = dy, 1 = x][row * 32 + unit]: kWgStages x 2 x 16 KB.
-__shared__ u32x4 g_wg_lds[kWgStages][2][kWgStep * 32];
+// 16-byte units of one token row of the dy tile, and of one stage (dy tile,
+// then x tile).
+template <int kMT>
+constexpr int kWgDyUnits = 8 * kMT;
+template <int kMT>
+constexpr int kWgStageUnits = kWgStep * (kWgDyUnits<kMT> + 32);
 
 // Byte offset (from its tile's base) of lane `lane`'s first transposed read
 // of fragment j: column 32j + lane % 32 of the wave's half h, token rows
@@ -97,41 +117,46 @@ __shared__ u32x4 g_wg_lds[kWgStages][2][kWgStep * 32];
 // i % 4 of the 8 bytes that lane 4e + i / 4 addresses, so lane 4e + c
 // addresses row e, columns 4c..4c+3 of the group's 16-column strip.  A second
 // read 4 rows lower completes the 8 tokens.
+template <int kUnits>
 __device__ __forceinline__ uint32_t wg_read_off(int lane, int h, int j) {
   const int l16 = lane & 15, e = l16 >> 2;
   const int row = 8 * (lane >> 5) + e;
-  const int u = 16 * h + 4 * j + 2 * ((lane >> 4) & 1) + ((l16 >> 1) & 1);
-  return (uint32_t)(512 * row + 16 * wg_unit(row, u) + 8 * (l16 & 1));
+  const int u = kUnits / 2 * h + 4 * j + 2 * ((lane >> 4) & 1) + ((l16 >> 1) & 1);
+  return (uint32_t)(16 * (kUnits * row + wg_unit(row, u)) + 8 * (l16 & 1));
 }
 
-// Fragment (8 tokens of one column, sub-step s) from the tile at `base`.
+// Fragment (8 tokens of one column, sub-step s) from the tile at `base`, whose
+// rows are kUnits 16-byte units long.
+template <int kUnits>
 __device__ __forceinline__ u32x4 wg_frag(const char *base, uint32_t off, int s) {
   typedef __attribute__((address_space(3))) char lds_char_t;
   typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
-  lds_char_t *p = (lds_char_t *)const_cast<char *>(base) + off + 8192 * s;
+  lds_char_t *p = (lds_char_t *)const_cast<char *>(base) + off + 256 * kUnits * s;
   const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t *)p);
-  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t *)(p + 2048));
+  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t *)(p + 64 * kUnits));
   const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
   return (u32x4){l2.x, l2.y, h2.x, h2.y};
 }
 
-// Fragment read q (0..7) of a sub-step in the order the sub-step's first
+// Fragment read q (0 .. kMT + 3) of a sub-step in the order the sub-step's first
 // MFMAs use them: dy0, x0, x1, x2, x3, dy1, dy2, dy3.
-__device__ __forceinline__ void wg_read(const char *tdy, const char *tx, const uint32_t (&rdy)[4],
-                                        const uint32_t (&rx)[4], u32x4 (&fd)[4], u32x4 (&fx)[4],
+template <int kMT>
+__device__ __forceinline__ void wg_read(const char *tdy, const char *tx, const uint32_t (&rdy)[kMT],
+                                        const uint32_t (&rx)[4], u32x4 (&fd)[kMT], u32x4 (&fx)[4],
                                         int s, int q) {
   if (q == 0 || q >= 5) {
     const int j = (q == 0) ? 0 : q - 4;
-    fd[j] = wg_frag(tdy, rdy[j], s);
+    fd[j] = wg_frag<kWgDyUnits<kMT>>(tdy, rdy[j], s);
   } else {
-    fx[q - 1] = wg_frag(tx, rx[q - 1], s);
+    fx[q - 1] = wg_frag<32>(tx, rx[q - 1], s);
   }
 }
 
-// One 32-token step t from stage `cur`: 2 sub-steps of 16 MFMAs.  The
+// One 32-token step t from stage `cur`: 2 sub-steps of 4 kMT MFMAs (the
+// counts below are kMT = 4's).  The
 // fragments of sub-step 1 are read (one per MFMA slot) during sub-step 0.
-// The 8 DMAs of this wave for step t + kWgStages - 1 (4 dy row pairs, 4 x
-// row pairs, two 256-column rows per instruction) go into stage `nxt` after
+// The kMT + 4 DMAs of this wave for step t + kWgStages - 1 (8 token rows of dy
+// and of x, 1 KB per instruction) go into stage `nxt` after
 // MFMAs 9, 11, .., 23 (the same DMAs in sub-step 0's first half measured
 // 1-2 % slower on 70B shapes); that stage held step t-1, whose reads all
 // ended before the barrier that closed step t-1.  The caller's barrier
@@ -143,47 +168,58 @@ __device__ __forceinline__ void wg_read(const char *tdy, const char *tx, const u
 // DMA after its slot's MFMA and reads.  The LDS stages come in as distinct
 // __restrict__ pointers: the compiler then knows that DMAs into `nxt` never
 // alias the reads of `cur` and waits (vmcnt) only at the barriers.
-__device__ __forceinline__ void wgrad_step(floatx16 (&acc)[4][4], u32x4 (&fd)[2][4],
+template <int kMT>
+__device__ __forceinline__ void wgrad_step(floatx16 (&acc)[kMT][4], u32x4 (&fd)[2][kMT],
                                            u32x4 (&fx)[2][4], const char *__restrict__ cur_dy,
                                            const char *__restrict__ cur_x,
                                            char *__restrict__ nxt_dy, char *__restrict__ nxt_x,
-                                           const uint32_t (&rdy)[4], const uint32_t (&rx)[4],
+                                           const uint32_t (&rdy)[kMT], const uint32_t (&rx)[4],
                                            __amdgpu_buffer_rsrc_t rs_dy, __amdgpu_buffer_rsrc_t rs_x,
-                                           uint32_t (&vdy)[4], uint32_t (&vx)[4],
+                                           uint32_t (&vdy)[kMT], uint32_t (&vx)[4],
                                            uint32_t step_dy, uint32_t step_x, bool more, int wave) {
-  // Previous step's last 8 MFMAs, then this step's sub-step 0 reads.
-  static_for<0, 8>([&](auto I) {
+  constexpr int kReads = kMT + 4, kDmas = kMT + 4;
+  constexpr int kPost = 2 * kMT;           // MFMAs that open the next step
+  constexpr int kFront = 8 * kMT - kPost;  // the others
+  // Previous step's last MFMAs, then this step's sub-step 0 reads.
+  static_for<0, kPost>([&](auto I) {
     constexpr int i = decltype(I)::value;
-    constexpr int mt = 2 + (i >> 2), nt = i & 3;
+    constexpr int mt = kMT / 2 + (i >> 2), nt = i & 3;
     acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
         __builtin_bit_cast(bf16x8, fx[1][nt]), __builtin_bit_cast(bf16x8, fd[1][mt]),
         acc[mt][nt], 0, 0, 0);
-    wg_read(cur_dy, cur_x, rdy, rx, fd[0], fx[0], 0, i);
+    static_for<0, kReads>([&](auto Q) {
+      constexpr int q = decltype(Q)::value;
+      if constexpr (q * kPost / kReads == i)
+        wg_read<kMT>(cur_dy, cur_x, rdy, rx, fd[0], fx[0], 0, q);
+    });
     __builtin_amdgcn_sched_barrier(0);
   });
-  static_for<0, 24>([&](auto N) {
+  static_for<0, kFront>([&](auto N) {
     constexpr int n = decltype(N)::value;
-    constexpr int s = n / 16, i = n % 16;
+    constexpr int s = n / (4 * kMT), i = n % (4 * kMT);
     constexpr int mt = i >> 2, nt = i & 3;
     acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
         __builtin_bit_cast(bf16x8, fx[s][nt]), __builtin_bit_cast(bf16x8, fd[s][mt]),
         acc[mt][nt], 0, 0, 0);
-    if constexpr (s == 0 && i < 8) wg_read(cur_dy, cur_x, rdy, rx, fd[1], fx[1], 1, i);
-    if constexpr (n >= 8 && (n & 1) == 1) {
-      // DMA d = (n - 8) / 2 after MFMAs 9, 11, .., 23: operand d / 4,
-      // instruction d % 4 (rows 8 wave + 2 (d % 4) and the next).
-      constexpr int d = (n - 8) / 2;
+    if constexpr (s == 0 && i < kReads)
+      wg_read<kMT>(cur_dy, cur_x, rdy, rx, fd[1], fx[1], 1, i);
+    // DMA d, after MFMAs 9, 11, .., 23 (kMT = 4) or 6, 7, .., 11 (kMT = 2): the
+    // kMT of dy, then the 4 of x.
+    constexpr int kGap = kMT / 2;
+    constexpr int back = kFront - 1 - n;  // MFMAs after this one
+    if constexpr (back % kGap == 0 && back / kGap < kDmas) {
+      constexpr int d = kDmas - 1 - back / kGap;
       if (more) {
-        if constexpr (d < 4) {
+        if constexpr (d < kMT) {
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              rs_dy, (lds_void_t *)(nxt_dy + 1024 * (4 * wave + d)), 16,
+              rs_dy, (lds_void_t *)(nxt_dy + 1024 * (kMT * wave + d)), 16,
               (int)vdy[d], 0, 0, 0);
           vdy[d] += step_dy;
         } else {
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              rs_x, (lds_void_t *)(nxt_x + 1024 * (4 * wave + d - 4)), 16, (int)vx[d - 4], 0, 0,
-              0);
-          vx[d - 4] += step_x;
+              rs_x, (lds_void_t *)(nxt_x + 1024 * (4 * wave + d - kMT)), 16, (int)vx[d - kMT], 0,
+              0, 0);
+          vx[d - kMT] += step_x;
         }
       }
     }
@@ -193,27 +229,28 @@ __device__ __forceinline__ void wgrad_step(floatx16 (&acc)[4][4], u32x4 (&fd)[2]
 
 // The barrier that closes step t: this wave's DMAs of step t+1 have landed
 // and every LDS read of step t has ended.  Its DMAs of the later steps in
-// the ring (t+2 .. t+kWgStages-1, 8 each, issued after t+1's, those that
+// the ring (t+2 .. t+kWgStages-1, kMT + 4 each, issued after t+1's, those that
 // exist) may still be in flight: vmcnt retires in issue order.
+template <int kMT>
 __device__ __forceinline__ void wgrad_close_step(int64_t t, int64_t nsteps) {
   int64_t later = nsteps - t - 2;  // steps after t+1 that exist, clamped below
   later = (later < 0) ? 0 : (later > kWgStages - 2) ? kWgStages - 2 : later;
   static_for<0, kWgStages - 1>([&](auto I) {
     constexpr int a = decltype(I)::value;  // exactly one a == later
-    if (later == a) step_barrier<8 * a>();
+    if (later == a) step_barrier<(kMT + 4) * a>();
   });
 }
 
 // Direct epilogue, for ragged columns and outputs without 16-byte stores: four
 // adjacent fp32 per store.
-template <bool kAcc>
-__device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[4][4], float *dw,
+template <bool kAcc, int kMT>
+__device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[kMT][4], float *dw,
                                          int64_t n0, int64_t k0, int64_t N, int lane,
                                          bool vec_ok) {
   asm volatile("" : "+v"(lane));  // as in wg_store_lds
   const int jl = lane & 31, grp = lane >> 5;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+  for (int mt = 0; mt < kMT; ++mt) {
     const int64_t n = n0 + 32 * mt + jl;
     if (n < N) {
       float *row = dw + n * g.K;
@@ -251,8 +288,8 @@ __device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&ac
 // 826 (909 -> 867).  Non-temporal stores: without them 367 us for 28672 x 8192
 // over 512 tokens.  Accumulating is its own instantiation: as a run-time test
 // it spilled 51 registers in both.
-template <bool kAcc>
-__device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 (&acc)[4][4],
+template <bool kAcc, int kMT>
+__device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 (&acc)[kMT][4],
                                              floatx4 *lds, float *dw, int64_t n0, int64_t k0,
                                              int64_t N, int lane) {
   // An opaque lane index keeps the per-lane addresses below from being hoisted
@@ -262,7 +299,7 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
   const int r0 = lane >> 5, c = lane & 31;  // read-back: row 2i + r0, chunk c
   // The wave's rows below N through a buffer resource that ends after the last.
   const int64_t left = N - n0;
-  const int64_t rows = left <= 0 ? 0 : (left > 128 ? 128 : left);
+  const int64_t rows = left <= 0 ? 0 : (left > 32 * kMT ? 32 * kMT : left);
   const uint32_t ld4 = (uint32_t)(g.K * 4);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
       (void *)(rows > 0 ? dw + n0 * g.K + k0 : dw), 0,
@@ -270,7 +307,7 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
   typedef unsigned int uvec4 __attribute__((ext_vector_type(4)));
   constexpr int kStoreNt = 2;  // non-temporal
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+  for (int mt = 0; mt < kMT; ++mt) {
     const uint32_t base = (uint32_t)(32 * mt + r0) * ld4 + 16u * (uint32_t)c;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt)
@@ -313,27 +350,27 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
   }
 }
 
-// One output tile: its 256 x 256 dW block over all M tokens.
-template <bool kAcc>
-__global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g) {
+// One output tile: its 64 kMT x 256 dW block over all M tokens.
+template <bool kAcc, int kMT>
+__global__ void __launch_bounds__(kWgThreads, 4 / kMT) wgrad_kernel(const WgradArgs g) {
   const int T = g.tiles_n * g.tiles_k;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int hn = wave >> 1, hk = wave & 1;  // the wave's halves of n and k
-  uint32_t rdy[4], rx[4];
+  __shared__ u32x4 lds[kWgStages][kWgStageUnits<kMT>];
+  uint32_t rdy[kMT], rx[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    rdy[j] = wg_read_off(lane, hn, j);
-    rx[j] = wg_read_off(lane, hk, j);
-  }
+  for (int j = 0; j < kMT; ++j) rdy[j] = wg_read_off<kWgDyUnits<kMT>>(lane, hn, j);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) rx[j] = wg_read_off<32>(lane, hk, j);
   char *ldy[kWgStages], *lx[kWgStages];
 #pragma unroll
   for (int i = 0; i < kWgStages; ++i) {
-    ldy[i] = reinterpret_cast<char *>(&g_wg_lds[i][0][0]);
-    lx[i] = reinterpret_cast<char *>(&g_wg_lds[i][1][0]);
+    ldy[i] = reinterpret_cast<char *>(&lds[i][0]);
+    lx[i] = reinterpret_cast<char *>(&lds[i][kWgStep * kWgDyUnits<kMT>]);
   }
   // 16 KB of the ring for each wave's epilogue.
-  floatx4 *lds_wave = reinterpret_cast<floatx4 *>(&g_wg_lds[0][0][0]) + 1024 * wave;
+  floatx4 *lds_wave = reinterpret_cast<floatx4 *>(&lds[0][0]) + 1024 * wave;
   const int64_t nsteps = (g.M + kWgStep - 1) / kWgStep;
   const uint32_t step_x = (uint32_t)(kWgStep * g.K * 2);
 #pragma unroll 1
@@ -350,7 +387,7 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
     int32_t t0 = g.tile0[0];
 #pragma unroll
     for (int j = 1; j < kMaxWgGroups; ++j) t0 = (gi == j) ? g.tile0[j] : t0;
-    const int64_t n0 = (int64_t)(tn - t0) * kWgTile, k0 = (int64_t)tk * kWgTile;
+    const int64_t n0 = (int64_t)(tn - t0) * (64 * kMT), k0 = (int64_t)tk * kWgTile;
     const uint32_t step_dy = (uint32_t)(kWgStep * N * 2);
     // Buffer resources based at the tiles' first columns; num_records ends
     // at the matrix end, so token rows >= M (and the last row's columns past
@@ -360,15 +397,21 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
         (void *)(dy + n0), 0, (int)(g.M * N * 2 - n0 * 2), kBufferFlags);
     const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(g.x + k0), 0, (int)(g.M * g.K * 2 - k0 * 2), kBufferFlags);
-    // Lane offsets of this wave's 4 DMAs per operand for step 0: instruction
-    // d writes rows 8 wave + 2d + (lane / 32), physical unit lane % 32.
-    uint32_t vdy[4], vx[4];
+    // Lane offsets of this wave's DMAs for step 0: x instruction d writes rows
+    // 8 wave + 2d + (lane / 32), physical unit lane % 32; of dy, whose rows are
+    // kWgDyUnits long, each writes 64 / kWgDyUnits rows.
+    uint32_t vdy[kMT], vx[4];
+    constexpr int kDyRows = 64 / kWgDyUnits<kMT>;
+#pragma unroll
+    for (int d = 0; d < kMT; ++d) {
+      const int r = 8 * wave + kDyRows * d + lane / kWgDyUnits<kMT>;
+      const int u = wg_unit(r, lane % kWgDyUnits<kMT>);  // the logical unit stored there
+      vdy[d] = (uint32_t)(r * N * 2 + 16 * u);
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int r = 8 * wave + 2 * d + (lane >> 5);
-      const int u = wg_unit(r, lane & 31);  // the logical unit stored at physical lane % 32
-      vdy[d] = (uint32_t)(r * N * 2 + 16 * u);
-      vx[d] = (uint32_t)(r * g.K * 2 + 16 * u);
+      vx[d] = (uint32_t)(r * g.K * 2 + 16 * wg_unit(r, lane & 31));
     }
     // Prologue: steps 0 .. kWgStages-2 (those that exist) into their
     // stages, then wait for step 0.
@@ -376,31 +419,33 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
     for (int p = 0; p < kWgStages - 1; ++p) {
       if (p < nsteps) {
 #pragma unroll
+        for (int d = 0; d < kMT; ++d) {
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              rs_dy, (lds_void_t *)(ldy[p] + 1024 * (kMT * wave + d)), 16, (int)vdy[d], 0, 0, 0);
+          vdy[d] += step_dy;
+        }
+#pragma unroll
         for (int d = 0; d < 4; ++d) {
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              rs_dy, (lds_void_t *)(ldy[p] + 1024 * (4 * wave + d)), 16, (int)vdy[d], 0, 0, 0);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(
               rs_x, (lds_void_t *)(lx[p] + 1024 * (4 * wave + d)), 16, (int)vx[d], 0, 0, 0);
-          vdy[d] += step_dy;
           vx[d] += step_x;
         }
       }
     }
-    wgrad_close_step(-1, nsteps);
+    wgrad_close_step<kMT>(-1, nsteps);
 
-    floatx16 acc[4][4];
+    floatx16 acc[kMT][4];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.0f;
-    u32x4 fd[2][4], fx[2][4];
+    u32x4 fd[2][kMT], fx[2][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      fd[1][i] = (u32x4){0u, 0u, 0u, 0u};
-      fx[1][i] = (u32x4){0u, 0u, 0u, 0u};
-    }
+    for (int i = 0; i < kMT; ++i) fd[1][i] = (u32x4){0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fx[1][i] = (u32x4){0u, 0u, 0u, 0u};
     // Step t computes from stage t % kWgStages and loads step
     // t + kWgStages - 1 into the stage before it.
     int64_t t = 0;
@@ -409,37 +454,37 @@ __global__ void __launch_bounds__(kWgThreads, 1) wgrad_kernel(const WgradArgs g)
       static_for<0, kWgStages>([&](auto I) {
         constexpr int i = decltype(I)::value;
         constexpr int c = i, nx = (i + kWgStages - 1) % kWgStages;
-        wgrad_step(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
+        wgrad_step<kMT>(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
                    step_dy, step_x, t + i + kWgStages - 1 < nsteps, wave);
-        wgrad_close_step(t + i, nsteps);
+        wgrad_close_step<kMT>(t + i, nsteps);
       });
     }
     static_for<0, kWgStages - 1>([&](auto I) {
       constexpr int i = decltype(I)::value;
       constexpr int c = i, nx = (i + kWgStages - 1) % kWgStages;
       if (t + i < nsteps) {
-        wgrad_step(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
+        wgrad_step<kMT>(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
                    step_dy, step_x, false, wave);
-        wgrad_close_step(t + i, nsteps);
+        wgrad_close_step<kMT>(t + i, nsteps);
       }
     });
-    // The last step's final 8 MFMAs.
+    // The last step's final MFMAs.
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int mt = 2 + (i >> 2), nt = i & 3;
+    for (int i = 0; i < 2 * kMT; ++i) {
+      const int mt = kMT / 2 + (i >> 2), nt = i & 3;
       acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
           __builtin_bit_cast(bf16x8, fx[1][nt]), __builtin_bit_cast(bf16x8, fd[1][mt]),
           acc[mt][nt], 0, 0, 0);
     }
 
-    // Epilogue.  Lane l holds dW row n = n0 + 128 hn + 32 mt + l % 32 and
+    // Epilogue.  Lane l holds dW row n = n0 + 32 kMT hn + 32 mt + l % 32 and
     // columns k = k0 + 128 hk + 32 nt + 8 j + 4 (l / 32) + i in registers
     // 4 j + i of tile [mt][nt].
     const bool vec_ok = ((reinterpret_cast<uintptr_t>(dw) & 15) == 0) && ((g.K & 3) == 0);
     if (vec_ok && k0 + kWgTile <= g.K && g.K < ((int64_t)1 << 22))  // 32-bit row offsets
-      wg_store_lds<kAcc>(g, acc, lds_wave, dw, n0 + 128 * hn, k0 + 128 * hk, N, lane);
+      wg_store_lds<kAcc, kMT>(g, acc, lds_wave, dw, n0 + 32 * kMT * hn, k0 + 128 * hk, N, lane);
     else
-      wg_store<kAcc>(g, acc, dw, n0 + 128 * hn, k0 + 128 * hk, N, lane, vec_ok);
+      wg_store<kAcc, kMT>(g, acc, dw, n0 + 32 * kMT * hn, k0 + 128 * hk, N, lane, vec_ok);
     // The next tile's prologue DMAs overwrite the LDS that the last step and
     // the epilogues read: every wave's reads (not its stores) end before this.
     step_barrier<63>();
@@ -450,6 +495,34 @@ __global__ void fill_zero_f32(float *__restrict__ p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     p[i] = 0.0f;
+}
+
+// dW rows per tile / 64: 4 (256-row tiles, one workgroup a CU) or 2 (128-row
+// tiles, two workgroups a CU).  Two workgroups hide one's stores and first
+// loads behind the other's products, and half tiles leave less of a last round
+// idle; but each x fragment feeds half the products.  The costs below are in
+// rounds of 256-row tiles, one per CU.  A full round of 128-row tiles (two a
+// CU) against it, 8192 x 8192: 256 tokens 57 us against 76, 1000 tokens 130
+// against 146, 2048 tokens 234 against 242, 4096 tokens 432 against 421, 8192
+// tokens 850 against 808; a round with one 128-row tile a CU takes 0.58-0.7.
+// 6000 x 3000 (1.1 rounds against 2) over 4096 tokens: 156 against 189 us;
+// 1024 x 8192 over 1000 tokens: 23 against 31; 1024 x 1024 over 1000: 15
+// against 25.
+// tiles4: 256-row tile rows of all products.  Called on sizes whose tile count
+// fits 31 bits (a 128-row tiling that would not keeps the 256-row one).
+static int wg_tile_mt(const int64_t *ns, int32_t count, int64_t m, int64_t tiles4,
+                      int64_t tiles_k) {
+  const int64_t cus = cu_slots();
+  int64_t tiles2 = 0;
+  for (int i = 0; i < count; ++i) tiles2 += (ns[i] + 127) / 128;
+  if (tiles2 * tiles_k > 0x7fffffff) return 4;
+  const int64_t t2 = tiles2 * tiles_k;
+  const double full = m <= 1024 ? 0.95 : (m <= 2048 ? 1.0 : 1.06);
+  const int64_t rest = t2 % (2 * cus);
+  const double cost2 = (double)(t2 / (2 * cus)) * full +
+                       (rest == 0 ? 0.0 : (rest <= cus ? 0.65 : full));
+  const double cost4 = (double)((tiles4 * tiles_k + cus - 1) / cus);
+  return cost2 < cost4 ? 2 : 4;
 }
 
 static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, float *const *dws,
@@ -515,14 +588,20 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
     g.dy[i] = dys[i];
     g.dw[i] = dws[i];
     g.N[i] = n;
-    g.tile0[i] = (int32_t)tiles_n;
-    tiles_n += (n + kWgTile - 1) / kWgTile;
+    tiles_n += (n + 255) / 256;
     if (tiles_n > 0x7fffffff) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
+  }
+  if (tiles_n * g.tiles_k > 0x7fffffff)
+    return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
+  const int mt = wg_tile_mt(ns, count, m, tiles_n, g.tiles_k);
+  tiles_n = 0;
+  for (int i = 0; i < count; ++i) {
+    g.tile0[i] = (int32_t)tiles_n;
+    tiles_n += (ns[i] + 64 * mt - 1) / (64 * mt);
   }
   for (int i = count; i <= kMaxWgGroups; ++i) g.tile0[i] = (int32_t)tiles_n;
   g.tiles_n = (int32_t)tiles_n;
   const int64_t T = tiles_n * g.tiles_k;
-  if (T > 0x7fffffff) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
   if (m == 0) {
     // An empty sum: dw += 0, or dw = 0 (a fill kernel rather than
     // hipMemsetAsync, so that a caller may capture the call in a HIP graph).
@@ -541,14 +620,21 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
   // XCD blocks (wg_map_tile) when every round is full: the squarest
   // blk_n x blk_k = G / 8 that divides the tile grid (the products' tile
   // rows stacked).
-  const int64_t G = persistent_grid(T);
+  const int64_t slots = (int64_t)cu_slots() * (4 / mt);
+  const int64_t G = T < slots ? T : slots;
+  // Strips of 8 tile columns; the 64 slots of an XCD with 128-row tiles read
+  // less per step from strips of 4, which pays once the steps outweigh the
+  // stores (28672 x 8192 over 256 tokens: 188 us with 8, 203 with 4; 2 x 11008
+  // x 4096 over 1000: 181 and 176, over 8192: 1289 and 1232).
+  g.strip = (mt == 2 && m > 512) ? 4 : 8;
+  if (g.strip > g.tiles_k) g.strip = g.tiles_k;
   if (G % 8 == 0 && T % G == 0) {
     const int S = (int)(G / 8);
     int best = 0;
     for (int bn = 1; bn <= S; ++bn) {
       if (S % bn != 0 || g.tiles_n % bn != 0 || g.tiles_k % (S / bn) != 0) continue;
       const int bk = S / bn;
-      const int cost = bn + bk;  // column blocks read per XCD and step
+      const int cost = mt * bn + 4 * bk;  // columns read per XCD and step, in 64s
       if (best == 0 || cost < best) {
         best = cost;
         g.blk_n = bn;
@@ -556,10 +642,9 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
       }
     }
   }
-  if (accumulate)
-    hipLaunchKernelGGL(wgrad_kernel<true>, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
-  else
-    hipLaunchKernelGGL(wgrad_kernel<false>, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
+  auto *kernel = mt == 4 ? (accumulate ? wgrad_kernel<true, 4> : wgrad_kernel<false, 4>)
+                         : (accumulate ? wgrad_kernel<true, 2> : wgrad_kernel<false, 2>);
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
   return check_launch("wgrad_kernel");
 }
 
