@@ -130,25 +130,30 @@ __device__ __forceinline__ uint32_t step_code(const uint2 *tab, float q, bool &n
   return t.y + ((q >= step) ? 1u : 0u);
 }
 
-// The lane's 8 elements e0 .. e0+7 (all below the limit): 16-byte loads.
+// The lane's 8 elements e0 .. e0+7 (all below the limit) as loaded: one 16-byte
+// load of bf16, two of fp32.
 template <typename T>
-__device__ __forceinline__ void load8_full(const T *__restrict__ x, int64_t e0, float v[8]) {
+struct Raw8 {
+  u32x4 w[sizeof(T) / 2];
+};
+template <typename T>
+__device__ __forceinline__ void load8_full(const T *__restrict__ x, int64_t e0, Raw8<T> &r) {
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(T) / 2; ++i) r.w[i] = *((const u32x4 *)(x + e0) + i);
+}
+
+template <typename T>
+__device__ __forceinline__ void unpack8(const Raw8<T> &r, float v[8]) {
   // Elements go through scalar temporaries: hipcc folds a bit_cast of a
   // vector-element subscript to element 0 for every index.
-  if constexpr (sizeof(T) == 4) {
-    const u32x4 a = *(const u32x4 *)(x + e0);
-    const u32x4 b = *(const u32x4 *)(x + e0 + 4);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t ak = a[k], bk = b[k];
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t ak = r.w[0][k];
+    if constexpr (sizeof(T) == 4) {
+      const uint32_t bk = r.w[1][k];
       v[k] = __builtin_bit_cast(float, ak);
       v[4 + k] = __builtin_bit_cast(float, bk);
-    }
-  } else {
-    const u32x4 a = *(const u32x4 *)(x + e0);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t ak = a[k];
+    } else {
       v[2 * k] = __builtin_bit_cast(float, ak << 16);
       v[2 * k + 1] = __builtin_bit_cast(float, ak & 0xffff0000u);
     }
@@ -259,7 +264,9 @@ __device__ __forceinline__ void quantize_tile_guarded(const T *__restrict__ x, i
 
 // Chunks of kU full tiles (x 16-byte and packed 4-byte aligned): one wave
 // takes chunks c0, c0 + dc, ... < nchunks, with the next chunk's loads
-// issued before the current chunk's codes (two register sets, alternating).
+// issued before the current chunk's codes (two register sets, alternating,
+// which hold x as loaded: unpacked at the load, bf16 waited for the next
+// chunk within the current one's codes).
 // Every path through a chunk issues the same loads and stores (all lanes
 // of a block store its absmax, the same value to the same address; the
 // loop's exits each get their own copy of the codes), so the wait before a
@@ -271,19 +278,23 @@ __device__ __forceinline__ void quantize_wave_full(const T *__restrict__ x, int6
                                                    AbsmaxOut absmax_out) {
   const int lane = threadIdx.x & 63;
   if (c0 >= nchunks) return;  // wave-uniform
-  float va[kU][8], vb[kU][8];
-  auto load = [&](float (&v)[kU][8], int64_t c) {
+  Raw8<T> va[kU], vb[kU];
+  auto load = [&](Raw8<T> (&v)[kU], int64_t c) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) load8_full<T>(x, tile_e0(c * kU + u) + 8 * lane, v[u]);
   };
-  auto emit = [&](float (&v)[kU][8], int64_t c) {
+  auto emit = [&](Raw8<T> (&r)[kU], int64_t c) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int64_t t = c * kU + u;
       const int64_t e0 = tile_e0(t) + 8 * lane;
       uint32_t word;
-      const float m = encode8<true, kLanes>(tab, v[u], e0, 0, word);
-      *(uint32_t *)(packed + (e0 >> 1)) = word;
+      float v[8];
+      unpack8<T>(r[u], v);
+      const float m = encode8<true, kLanes>(tab, v, e0, 0, word);
+      // Non-temporal (with the default policy, 28672 x 8192: fp32 208 against
+      // 198 us; bf16 with double-quant 115 against 109).
+      __builtin_nontemporal_store(word, (uint32_t *)(packed + (e0 >> 1)));
       absmax_out(t, lane >> kLanes, m);
     }
   };
@@ -654,6 +665,11 @@ static int32_t dequant_batch(const nf4s_tensor *ts, const int64_t *ns, uint16_t 
 
 constexpr int kQuantU = 1;         // tiles per chunk
 constexpr int kQuantMaxGrid = 1024;  // workgroups of the quantize launches
+// Tiles per chunk with double-quant: 2 KB of x in flight per wave, one tile of
+// fp32 or two of bf16.  28672 x 8192 bf16 with one tile 114-119 us, two 109;
+// fp32 with one 200, two 204.
+template <typename T>
+constexpr int kQuantDqU = sizeof(T) == 4 ? 1 : 2;
 
 template <typename T>
 static bool quantize_vec_ok(const T *x, const uint8_t *packed) {
@@ -694,7 +710,7 @@ static int32_t quantize_dq(const T *x, int64_t n, int32_t block_size, int32_t gr
   const size_t lds = (size_t)group * sizeof(float);
   const uint32_t grid = (uint32_t)(ng < kQuantMaxGrid ? ng : kQuantMaxGrid);
   if (quantize_vec_ok(x, packed))
-    hipLaunchKernelGGL((quantize_dq_kernel<T, true, kQuantU>), dim3(grid), dim3(256), lds,
+    hipLaunchKernelGGL((quantize_dq_kernel<T, true, kQuantDqU<T>>), dim3(grid), dim3(256), lds,
                        as_stream(stream), x, n, group, packed, q, scale, nb, ng);
   else
     hipLaunchKernelGGL((quantize_dq_kernel<T, false, kQuantU>), dim3(grid), dim3(256), lds,
