@@ -134,7 +134,7 @@ __device__ __forceinline__ void sk_step(floatx16 (&acc)[TM], const SkBlock &blk,
   auto read_x = [&](int j, u32x4 (&xf)[TM]) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
-      xf[tm] = xt[sk_unit((32 * tm + jl) & (TR - 1), 8 * g + j)];
+      xf[tm] = xt[sk_unit(TR < 32 ? jl & (TR - 1) : 32 * tm + jl, 8 * g + j)];
   };
   uint32_t o[2][4];
   {
@@ -181,11 +181,11 @@ __device__ __forceinline__ bool sk_vec_ok(const uint16_t *out, int64_t ldo) {
   return ((reinterpret_cast<uintptr_t>(out) & 7) == 0) && ((ldo & 3) == 0);
 }
 
-// TR: token rows in LDS (4, 16, 32, 64, 128 >= m).  SwiGLU: even waves of a
+// TR: token rows in LDS (4, 16, 32, 64, 96, 128 >= m).  SwiGLU: even waves of a
 // k-group take 32 gate rows, odd ones the same 32 up rows, and hidden is
 // elementwise between their partial tiles.
 template <int TR, int WN, int WK, bool kSwiglu, bool kDQ>
-__global__ void __launch_bounds__(64 * WN * WK, TR < 128 ? 4 : 2) nf4_skinny_kernel(const SkinnyArgs a) {
+__global__ void __launch_bounds__(64 * WN * WK, TR <= 64 ? 4 : 2) nf4_skinny_kernel(const SkinnyArgs a) {
   static_assert(!kSwiglu || WN % 2 == 0, "gate and up rows in pairs of waves");
   constexpr int TM = TR < 32 ? 1 : TR / 32;
   constexpr int kCols = 32 * (kSwiglu ? WN / 2 : WN);  // output columns of the workgroup
@@ -403,6 +403,9 @@ __global__ void __launch_bounds__(256) nf4_skinny_sum_kernel(const SkinnyArgs a,
 // 96, 4096 x 4096 21 against 25; 512-row tiles took 175 and 42).  Beyond them
 // the wave has no registers for more tokens: the tiled kernel, whose waves
 // share the dequantized weights instead, takes over.
+// 96-token tiles (96 KB) between: the MFMAs and x reads of a quarter fewer token
+// tiles; at 80 tokens against 128-token ones 28672 x 8192 84.2 -> 76.2 us,
+// 4096 x 4096 19.4 -> 17.9, SwiGLU of 13824 x 5120 52.5 -> 47.2.
 struct SkShape {
   int tr, wn, wk;
 };
@@ -411,6 +414,7 @@ static SkShape sk_shape(int64_t m, bool swiglu) {
   if (m <= 16) return swiglu ? SkShape{16, 2, 4} : SkShape{16, 1, 8};
   if (m <= 32) return {32, 2, 4};
   if (m <= 64) return {64, 4, 2};
+  if (m <= 96) return {96, 4, 2};
   return {128, 4, 2};
 }
 
@@ -418,7 +422,7 @@ static SkShape sk_shape(int64_t m, bool swiglu) {
 // CU take at once, each wave keeping at least 4 steps (fewer would spend more
 // on the partials than on the weights).
 static int sk_slices(int64_t tiles, int64_t steps, const SkShape &sh) {
-  const int64_t slots = (sh.tr == 128 ? 1 : 2) * (int64_t)cu_slots();  // 128 or 64 KB of LDS
+  const int64_t slots = (sh.tr > 64 ? 1 : 2) * (int64_t)cu_slots();  // 96 KB of LDS or more: one
   int64_t s = slots / tiles;
   const int64_t most = steps / (4 * sh.wk);  // at least 4 steps per wave
   if (s > most) s = most;
@@ -461,6 +465,7 @@ static void sk_launch(const SkinnyArgs &a, const SkShape &sh, uint32_t grid, hip
       break;
     case 32: hipLaunchKernelGGL((nf4_skinny_kernel<32, 2, 4, kSwiglu, kDQ>), g, b, 0, s, a); break;
     case 64: hipLaunchKernelGGL((nf4_skinny_kernel<64, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
+    case 96: hipLaunchKernelGGL((nf4_skinny_kernel<96, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
     default: hipLaunchKernelGGL((nf4_skinny_kernel<128, 4, 2, kSwiglu, kDQ>), g, b, 0, s, a); break;
   }
 }
