@@ -41,3 +41,20 @@ def test_fwd(m, n, k, dq):
     print(f"m={m} n={n} k={k} dq={dq}", flush=True)
     assert torch.equal(gemm.linear_fwd(x, w), ref)
     assert torch.equal(gemm.linear_fwd(x, w, split_k=False), ref)
+
+
+# Hidden widths on both sides of the line between 32- and 64-column tiles (the
+# wide ones with a ragged last tile).  fp32 silu on the gate sum: one bf16
+# rounding of the output, 2^-8 at most, and the hardware exponential and
+# reciprocal, a few fp32 ulps (below 1e-5).
+@pytest.mark.parametrize("m", [33, 64, 65, 96, 100, 128])
+@pytest.mark.parametrize("ff", [33, 8192, 8200, 20000])
+@pytest.mark.parametrize("k,dq", [(64, True), (448, False), (1024, True)])
+def test_swiglu_tile_widths(m, ff, k, dq):
+    wg, wu = _weight(ff, k, 1, dq), _weight(ff, k, 2, dq)
+    x, a, b = _two_hot(m, k)
+    gate = _sum(wg, a, b).double()
+    ref = gate * torch.sigmoid(gate) * _sum(wu, a, b).double()
+    print(f"m={m} ff={ff} k={k} dq={dq}", flush=True)
+    err = (gemm.linear_swiglu(x, wg, wu).double() - ref).abs()
+    assert (err <= ref.abs() * (2.0 ** -8 + 1e-5)).all(), (err / ref.abs()).max().item()
