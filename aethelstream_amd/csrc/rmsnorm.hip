@@ -12,8 +12,8 @@
 // meet in a tree, so rms can differ from the sequential sum in its last bits.
 //
 // The kernel is HBM-bound (4 bytes read and 2 written per element), one
-// workgroup per row.  The model widths (4096, 8192, 16384) keep the row in
-// registers between the reduction and the output; other widths read it twice.
+// workgroup per row.  Rows of 4096 to 16384 elements stay in registers between
+// the reduction and the output; others are read twice.
 #include "abi_common.hpp"
 #include "gemm_common.hpp"
 #include "nf4_device.hpp"
@@ -50,21 +50,31 @@ __device__ __forceinline__ u32x2 norm_chunk(const floatx4 &v, const floatx4 &g, 
   return (u32x2){pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
 }
 
-// d = 1024 * kChunks: the row stays in registers between the two passes
-// (thread t holds 4-element chunks t, t + 256, ...), so x is read once.
-template <int kChunks>
+// d <= 1024 * kChunks (kWhole: equal): the row stays in registers between the
+// two passes (thread t holds 4-element chunks t, t + 256, ..., those below
+// d / 4; an absent one adds +0 to its sum of squares), so x is read once, with
+// all its loads in flight.  8192 rows against the two-pass kernel below: 5120
+// wide 54.0 -> 44.0 us (5.7 TB/s), 7168 79.6 -> 61.3, 13824 163 -> 116.
+template <int kChunks, bool kWhole>
 __global__ void __launch_bounds__(kNormThreads) rmsnorm_fwd_reg_kernel(const float *__restrict__ x,
                                                                       const float *__restrict__ w,
-                                                                      float eps,
+                                                                      int64_t width, float eps,
                                                                       uint16_t *__restrict__ y,
                                                                       float *__restrict__ rms) {
   __shared__ float part[kNormThreads / 64];
-  constexpr int64_t d = 1024 * kChunks;
+  const int64_t d = kWhole ? 1024 * kChunks : width;
+  const int chunks = (int)(d >> 2);
+  auto present = [&](int c) {
+    return kWhole || (int)threadIdx.x + c * kNormThreads < chunks;
+  };
   const int64_t row = blockIdx.x;
   const floatx4 *xr = reinterpret_cast<const floatx4 *>(x + row * d) + threadIdx.x;
   floatx4 v[kChunks];
 #pragma unroll
-  for (int c = 0; c < kChunks; ++c) v[c] = __builtin_nontemporal_load(xr + c * kNormThreads);
+  for (int c = 0; c < kChunks; ++c) {
+    v[c] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+    if (present(c)) v[c] = __builtin_nontemporal_load(xr + c * kNormThreads);
+  }
   float s = 0.0f;
 #pragma unroll
   for (int c = 0; c < kChunks; ++c)
@@ -80,7 +90,9 @@ __global__ void __launch_bounds__(kNormThreads) rmsnorm_fwd_reg_kernel(const flo
   u32x2 *yr = reinterpret_cast<u32x2 *>(y + row * d) + threadIdx.x;
 #pragma unroll
   for (int c = 0; c < kChunks; ++c)
-    __builtin_nontemporal_store(norm_chunk(v[c], wr[c * kNormThreads], r), yr + c * kNormThreads);
+    if (present(c))
+      __builtin_nontemporal_store(norm_chunk(v[c], wr[c * kNormThreads], r),
+                                  yr + c * kNormThreads);
 }
 
 // Any d % 4 == 0: pass 1 sums the squares, pass 2 reads the row again (an L2
@@ -137,12 +149,22 @@ int32_t nf4s_rmsnorm_fwd(const float *x, const float *w, int64_t m, int64_t d, f
     return fail(NF4S_ERR_MISALIGNED, "x and w must be 16-byte aligned, y 8-byte aligned");
   hipStream_t s = as_stream(stream);
   const dim3 grid((uint32_t)m), block(kNormThreads);
-  switch (d) {
-    case 4096: hipLaunchKernelGGL(rmsnorm_fwd_reg_kernel<4>, grid, block, 0, s, x, w, eps, y, rms); break;
-    case 8192: hipLaunchKernelGGL(rmsnorm_fwd_reg_kernel<8>, grid, block, 0, s, x, w, eps, y, rms); break;
-    case 16384: hipLaunchKernelGGL(rmsnorm_fwd_reg_kernel<16>, grid, block, 0, s, x, w, eps, y, rms); break;
-    default: hipLaunchKernelGGL(rmsnorm_fwd_kernel, grid, block, 0, s, x, w, d, eps, y, rms); break;
+  // Rows of up to 4096 elements other than 4096 gain nothing from registers
+  // (8192 rows of 3000: 28 us against 27, of 1024: 10.7 against 12.4).
+  auto *kernel = rmsnorm_fwd_kernel;
+  switch ((d + 1023) / 1024) {
+    case 5: kernel = rmsnorm_fwd_reg_kernel<5, false>; break;
+    case 6: kernel = rmsnorm_fwd_reg_kernel<6, false>; break;
+    case 7: kernel = rmsnorm_fwd_reg_kernel<7, false>; break;
+    case 8: kernel = rmsnorm_fwd_reg_kernel<8, false>; break;
+    case 9: case 10: case 11: case 12: kernel = rmsnorm_fwd_reg_kernel<12, false>; break;
+    case 13: case 14: case 15: case 16: kernel = rmsnorm_fwd_reg_kernel<16, false>; break;
+    default: break;
   }
+  if (d == 4096) kernel = rmsnorm_fwd_reg_kernel<4, true>;
+  if (d == 8192) kernel = rmsnorm_fwd_reg_kernel<8, true>;
+  if (d == 16384) kernel = rmsnorm_fwd_reg_kernel<16, true>;
+  hipLaunchKernelGGL(kernel, grid, block, 0, s, x, w, d, eps, y, rms);
   return check_launch("rmsnorm_fwd_kernel");
 }
 
