@@ -87,7 +87,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void *p, int32_t
 // Loads the lane's block of the step that starts at block b (uniform).  A
 // step past the wave's range (!live, uniform) and a lane without a block
 // (past: the second one of a step that has only one) get zero words and a
-// zero absmax.
+// zero absmax: code and scale both, since the blocks that follow belong to
+// other rows, and an infinite or NaN scale of theirs times a zero code would
+// put NaN into this row.
 template <bool kDQ>
 __device__ __forceinline__ void sk_load(const SkRow &r, int b, bool live, bool past, SkBlock &v) {
   const uint32_t off = past ? kPast : r.poff;
@@ -101,8 +103,9 @@ __device__ __forceinline__ void sk_load(const SkRow &r, int b, bool live, bool p
   if constexpr (kDQ) {
     v.q = __builtin_amdgcn_raw_buffer_load_b8(am, (int)(past ? kPast : blk), 0, 0);
     const uint32_t sc = (r.sidx + (uint32_t)(b >> r.block_shift)) >> r.group_shift;
-    const uint32_t sv = __builtin_amdgcn_raw_buffer_load_b32(sk_rsrc(r.scale, r.scale_bytes),
-                                                             (int)(4 * sc), 0, 0);
+    const __amdgpu_buffer_rsrc_t rs = sk_rsrc(r.scale, live ? r.scale_bytes : 0);
+    const uint32_t sv = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(past ? kPast : 4 * sc), 0,
+                                                             0);
     v.s = __builtin_bit_cast(float, sv);
   } else {
     const uint32_t av = __builtin_amdgcn_raw_buffer_load_b32(am, (int)(past ? kPast : 4 * blk), 0,
