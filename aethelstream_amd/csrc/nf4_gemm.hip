@@ -29,8 +29,9 @@ static int32_t check_gemm(const uint16_t *act, const nf4s_tensor *w, int64_t m, 
   if (m < 0 || wn <= 0 || wk <= 0)
     return fail(NF4S_ERR_INVALID_ARGUMENT, "bad GEMM shape m=%lld n=%lld k=%lld",
                 (long long)m, (long long)wn, (long long)wk);
-  // Tile counts are 32-bit: (dim + 511) / 512 must fit before the launch
-  // code bounds the tile total.
+  // Keeps the tile counts of each dimension (at least 64 rows or columns a
+  // tile) and their sums over four weights far inside 64 bits; plan_launch
+  // bounds their product.
   constexpr int64_t kMaxDim = (int64_t)1 << 39;
   if (m > kMaxDim || wn > kMaxDim || wk > kMaxDim)
     return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "GEMM dimension beyond 2^39: m=%lld n=%lld k=%lld",
@@ -162,12 +163,13 @@ static int32_t gemm_fwd_groups(const uint16_t *x, const nf4s_tensor *ws, const i
       GemmGroup q = group_of(ws[j], ns[j]);
       q.out = ys[j];
       q.ldo = ns[j];
-      q.tiles_o = (int32_t)((ns[j] + kTileO - 1) / kTileO);
-      tiles += q.tiles_o;
+      const int64_t tiles_o = (ns[j] + kTileO - 1) / kTileO;
+      tiles += tiles_o;
+      if (tiles > kMaxTiles) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
+      q.tiles_o = (int32_t)tiles_o;
       ga.grp[ga.ngroups++] = q;
       done[j] = true;
     }
-    if (tiles > 0x7fffffff) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
     ga.tiles_o = (int32_t)tiles;
     rc = launch_fwd(ga, (kind[i] & 1) != 0, (kind[i] & 2) != 0, s, work, work_bytes);
     if (rc != NF4S_OK) return rc;
@@ -216,7 +218,7 @@ static int32_t gemm_swiglu(const uint16_t *x, const nf4s_tensor *wg, const nf4s_
   g.R = k;
   g.wk = k;
   const int64_t tiles_h = (ff + kTileO / 2 - 1) / (kTileO / 2);
-  if (tiles_h > 0x7fffffff) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
+  if (tiles_h > kMaxTiles) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
   ga.tiles_o = (int32_t)tiles_h;
   ga.grp[0] = group_of(*wg, ff);
   ga.grp[1] = group_of(*wu, ff);
@@ -253,7 +255,9 @@ static int32_t gemm_dgrad_groups(const uint16_t *const *dys, const nf4s_tensor *
   g.M = m;
   g.O = k;
   g.wk = k;
-  g.tiles_o = (int32_t)((k + kTileO - 1) / kTileO);
+  const int64_t tiles_o = (k + kTileO - 1) / kTileO;
+  if (tiles_o > kMaxTiles) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
+  g.tiles_o = (int32_t)tiles_o;
   for (int32_t i = 0; i < count; ++i) {
     GemmGroup q = group_of(ws[i], ns[i]);
     q.a = dys[i];

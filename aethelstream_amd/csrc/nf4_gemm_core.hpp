@@ -1620,10 +1620,13 @@ inline SplitPlan split_plan(int64_t T, int64_t nsteps, int unroll, int64_t slots
   return p;
 }
 
+// Largest tile count of a launch: the kernels count tiles in 32 bits.
+constexpr int64_t kMaxTiles = 0x7fffffff;
+
 // How a launch of m rows, `tiles_o` output tiles and `nsteps` reduction steps
 // runs: the rows per wave (32 kmt) and the split of its last round.
 struct LaunchPlan {
-  int kmt;
+  int kmt;  // 0: more than kMaxTiles tiles at every size
   int64_t tiles_m;
   SplitPlan split;
   int64_t bytes;  // workspace
@@ -1651,7 +1654,11 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
     LaunchPlan p{};
     p.kmt = kmt;
     p.tiles_m = (m + tile_m(kmt) - 1) / tile_m(kmt);
-    const int64_t T = p.tiles_m * tiles_o, slots = launch_slots(kmt);
+    // With dimensions up to 2^39 the product of the tile counts passes 64
+    // bits; a size with too many tiles is no candidate.
+    int64_t T;
+    if (__builtin_mul_overflow(p.tiles_m, tiles_o, &T) || T > kMaxTiles) continue;
+    const int64_t slots = launch_slots(kmt);
     p.split = may_split ? split_plan(T, nsteps, unroll, slots) : SplitPlan{0, 1, 0};
     p.bytes = p.split.tail_tiles * p.split.splits * partial_floats(kmt) * (int64_t)sizeof(float);
     const int64_t r = T % slots;
@@ -1661,7 +1668,7 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
             kFixupUsPerMiB * (double)(p.bytes >> 20);
     else if (r > 0)
       us += (kmt == 1 && 2 * r <= slots ? kSingleUs : kStepUs[kmt]) * nsteps + kRoundUs;
-    if (kmt == 4 || us < best_us) {
+    if (best.kmt == 0 || us < best_us) {
       best = p;
       best_us = us;
     }
@@ -1672,7 +1679,9 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
 // Workspace that is enough for the plan of these sizes, and for the split of
 // 512-row tiles, which callers size it by.
 inline int64_t plan_bytes(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll) {
-  const int64_t chosen = plan_launch(m, tiles_o, nsteps, unroll, true).bytes;
+  const LaunchPlan best = plan_launch(m, tiles_o, nsteps, unroll, true);
+  if (best.kmt == 0) return 0;
+  const int64_t chosen = best.bytes;
   const SplitPlan p = split_plan((m + tile_m(4) - 1) / tile_m(4) * tiles_o, nsteps, unroll,
                                  launch_slots(4));
   const int64_t whole = p.tail_tiles * p.splits * partial_floats(4) * (int64_t)sizeof(float);
@@ -1691,8 +1700,8 @@ inline LaunchPlan plan_with(int64_t m, int64_t tiles_o, int64_t nsteps, int unro
 // Fills in the launch's tiles and split; returns its work units, or -1 when
 // there are too many tiles.
 inline int64_t apply_plan(GroupedArgs &ga, const LaunchPlan &p, int64_t tiles_o, void *ws) {
+  if (p.kmt == 0) return -1;
   const int64_t T = p.tiles_m * tiles_o;
-  if (T > 0x7fffffff) return -1;
   ga.base.tiles_m = (int32_t)p.tiles_m;
   ga.full_tiles = (int32_t)(T - p.split.tail_tiles);
   ga.splits = (int32_t)p.split.splits;

@@ -225,3 +225,34 @@ def test_huge_sizes_are_rejected_not_wrapped():
     assert size.value == 0
     assert lib.nf4s_gemm_fwd_workspace_size(ns, 1, 1 << 62, 8192, ctypes.byref(size)) == 0
     assert size.value == 0
+
+
+def test_tile_counts_past_32_bits_are_refused_by_every_gemm():
+    """Dimensions up to 2^39 are valid one by one; a product of their tile
+    counts past 2^31 (with 128-row tiles up to 2^66, which wraps 64 bits to
+    zero or to a small number) is refused before any launch, and the workspace
+    queries report no split for it."""
+    lib = _lib.load()
+    x, out, top = 0x1000, 0x2000, 1 << 39
+    d = _desc(packed_len=1 << 62, absmax_len=1 << 56, bs=64)
+    p = ctypes.byref(d)
+    unsupported = _lib.NF4S_ERR_UNSUPPORTED_SHAPE
+    for m, n in ((top, top), (top - 128, 128 * 500), (1 << 31, 1 << 31)):
+        print(m, n, flush=True)
+        assert lib.nf4s_gemm_fwd(x, p, m, n, 64, out, None) == unsupported
+        assert b"too many tiles" in lib.nf4s_last_error_message()
+        assert lib.nf4s_gemm_fwd_swiglu(x, p, p, m, n, 64, out, None) == unsupported
+        assert lib.nf4s_gemm_dgrad(x, p, m, 64, n, out, None) == unsupported
+        assert b"too many tiles" in lib.nf4s_last_error_message()
+    # 2^32 tile columns alone.
+    assert lib.nf4s_gemm_dgrad(x, p, 1, 64, top, out, None) == unsupported
+    size = ctypes.c_int64(-1)
+    for ns in ([top], [top, 128 * 500], [top] * 4):
+        arr = (ctypes.c_int64 * len(ns))(*ns)
+        for m in (top, top - 128):
+            print(m, ns, flush=True)
+            assert lib.nf4s_gemm_fwd_workspace_size(arr, len(ns), m, 1024, ctypes.byref(size)) == 0
+            assert size.value == 0
+    arr = (ctypes.c_int64 * 1)(1 << 22)
+    assert lib.nf4s_gemm_dgrad_workspace_size(arr, 1, top, top, ctypes.byref(size)) == 0
+    assert size.value == 0
