@@ -1632,24 +1632,51 @@ struct LaunchPlan {
   int64_t bytes;  // workspace
 };
 
-// The row-block size whose rounds take the least time, from what a round
-// measured (K = 8192, weights from HBM, forward / input gradient, whole rounds
-// without a split): 1.66 / 1.71 us per 64-deep step for kMT = 4, 1.30 / 1.37
-// for 3, 1.02 / 1.09 for 2; for kMT = 1 1.30 with two workgroups a CU, 0.80
-// with one.  Larger tiles cost less per row (the dequantization and the
-// weight fragment reads serve more of them), smaller ones leave fewer rows
-// and CUs idle.  A round adds about 5 us (prologue and output burst), a split
-// its partials (0.3 us per MiB written and read) and a launch.  Against
-// 512-row tiles for everything, same box: forward 28672 x 8192 at 256 tokens
+// Time of a 64-deep step of a round in which `busy` of the `slots` workgroups
+// that the chip runs at once have a tile, in us: measured at K = 1024 to 28672
+// (weights from HBM, forward and input gradient alike) on a nearly idle chip,
+// at half the slots and at all of them, straight lines between.  Fewer
+// workgroups share the caches, the memory and the power: 172 tiles of 512 rows
+// on 256 CUs take 1.28 us a step where 256 take 1.66, and a plan that
+// charged the full step preferred 258 tiles of 384 rows for them (777 tokens,
+// 11008 x 4096: 99 us against 84).  With kMT = 1 the second half of the slots
+// is a second workgroup on each CU: one step more is then a step of two.
+inline double step_us(int kmt, int64_t busy, int64_t slots) {
+  constexpr double kIdle[5] = {0, 0.45, 0.70, 0.88, 0.98};
+  constexpr double kHalf[5] = {0, 0.78, 0.80, 1.04, 1.18};
+  constexpr double kPast[5] = {0, 0.95, 0.80, 1.04, 1.18};  // just past half
+  constexpr double kFull[5] = {0, 1.30, 1.02, 1.32, 1.66};
+  const double f = 2.0 * (double)busy / (double)slots;
+  return f <= 1.0 ? kIdle[kmt] + (kHalf[kmt] - kIdle[kmt]) * f
+                  : kPast[kmt] + (kFull[kmt] - kPast[kmt]) * (f - 1.0);
+}
+
+// The row-block size, with or without a split of its last round, whose rounds
+// take the least time.  Larger tiles cost less per row (the dequantization and
+// the weight fragment reads serve more of them), smaller ones leave fewer rows
+// and CUs idle.  A round adds about 5 us (prologue and output burst); a split
+// round 8 to 12.5 for that, short slices and the second launch, and its
+// partials (0.25 us per MiB written and read); 512-row tiles get 2 %, about
+// what the sums err by over several rounds.  Over 1010 shapes (128 to 8192
+// rows, 4 to 256 output tiles, K = 512 to 28672, both directions, widths that
+// take 16-byte stores and not) the choice takes 0.6 % more time than the best
+// of the eight on average, and nowhere more than 2 % over 512-row tiles.
+// Against those for everything, same box: forward 28672 x 8192 at 256 tokens
 // 178 -> 143 us, 384 tokens 195 -> 180 us; 8192 x 8192 at 256 tokens 66 -> 49
 // us; input gradient of 8192 x 8192 at 128 tokens 81 -> 39 us.
 inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll,
                               bool may_split) {
-  constexpr double kStepUs[5] = {0, 1.30, 1.02, 1.32, 1.66};
-  constexpr double kSingleUs = 0.80;  // kMT = 1, one workgroup a CU
-  constexpr double kRoundUs = 5.0, kFixupUs = 3.0, kFixupUsPerMiB = 0.3;
+  constexpr double kRoundUs = 5.0, kPartialUsPerMiB = 0.25;
+  constexpr double kSplitUs[5] = {0, 8.0, 10.5, 9.0, 12.5};
   LaunchPlan best{};
   double best_us = 0;
+  auto offer = [&](const LaunchPlan &p, double us) {
+    if (p.kmt == 4) us *= 0.98;
+    if (best.kmt == 0 || us < best_us) {
+      best = p;
+      best_us = us;
+    }
+  };
   for (int kmt = 4; kmt >= 1; --kmt) {
     LaunchPlan p{};
     p.kmt = kmt;
@@ -1658,20 +1685,25 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
     // bits; a size with too many tiles is no candidate.
     int64_t T;
     if (__builtin_mul_overflow(p.tiles_m, tiles_o, &T) || T > kMaxTiles) continue;
-    const int64_t slots = launch_slots(kmt);
-    p.split = may_split ? split_plan(T, nsteps, unroll, slots) : SplitPlan{0, 1, 0};
-    p.bytes = p.split.tail_tiles * p.split.splits * partial_floats(kmt) * (int64_t)sizeof(float);
-    const int64_t r = T % slots;
-    double us = (double)(T / slots) * (kStepUs[kmt] * nsteps + kRoundUs);
-    if (p.split.tail_tiles > 0)
-      us += kStepUs[kmt] * p.split.split_steps + kRoundUs + kFixupUs +
-            kFixupUsPerMiB * (double)(p.bytes >> 20);
-    else if (r > 0)
-      us += (kmt == 1 && 2 * r <= slots ? kSingleUs : kStepUs[kmt]) * nsteps + kRoundUs;
-    if (best.kmt == 0 || us < best_us) {
-      best = p;
-      best_us = us;
+    const int64_t slots = launch_slots(kmt), r = T % slots;
+    const double whole =
+        (double)(T / slots) * (step_us(kmt, slots, slots) * nsteps + kRoundUs);
+    double unsplit = whole + (r > 0 ? step_us(kmt, r, slots) * nsteps + kRoundUs : 0.0);
+    p.split = split_plan(T, nsteps, unroll, slots);
+    if (p.split.tail_tiles > 0) {
+      const int64_t tail = p.split.tail_tiles * p.split.splits;
+      p.bytes = tail * partial_floats(kmt) * (int64_t)sizeof(float);
+      const double split = whole + step_us(kmt, tail, slots) * p.split.split_steps +
+                           kSplitUs[kmt] + kPartialUsPerMiB * (double)(p.bytes >> 20);
+      if (may_split) offer(p, split);
+      // After whole rounds the slices are never the slower way: they also
+      // halve the output burst of rows that don't take 16-byte stores (830 x
+      // 36497 over K = 2048: 215 us split, 234 not).
+      if (T > slots && unsplit < split) unsplit = split;
     }
+    p.split = SplitPlan{0, 1, 0};
+    p.bytes = 0;
+    offer(p, unsplit);
   }
   return best;
 }
