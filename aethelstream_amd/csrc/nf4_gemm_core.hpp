@@ -1664,8 +1664,11 @@ inline double step_us(int kmt, int64_t busy, int64_t slots) {
 // Against those for everything, same box: forward 28672 x 8192 at 256 tokens
 // 178 -> 143 us, 384 tokens 195 -> 180 us; 8192 x 8192 at 256 tokens 66 -> 49
 // us; input gradient of 8192 x 8192 at 128 tokens 81 -> 39 us.
+// Only splits whose partials fit in ws_bytes of workspace are candidates; the
+// others' costs do not depend on it, so a call with the plan_bytes of its
+// sizes, or more, runs the plan they stand for.
 inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll,
-                              bool may_split) {
+                              int64_t ws_bytes) {
   constexpr double kRoundUs = 5.0, kPartialUsPerMiB = 0.25;
   constexpr double kSplitUs[5] = {0, 8.0, 10.5, 9.0, 12.5};
   LaunchPlan best{};
@@ -1695,7 +1698,7 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
       p.bytes = tail * partial_floats(kmt) * (int64_t)sizeof(float);
       const double split = whole + step_us(kmt, tail, slots) * p.split.split_steps +
                            kSplitUs[kmt] + kPartialUsPerMiB * (double)(p.bytes >> 20);
-      if (may_split) offer(p, split);
+      if (p.bytes <= ws_bytes) offer(p, split);
       // After whole rounds the slices are never the slower way: they also
       // halve the output burst of rows that don't take 16-byte stores (830 x
       // 36497 over K = 2048: 215 us split, 234 not).
@@ -1708,25 +1711,9 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
   return best;
 }
 
-// Workspace that is enough for the plan of these sizes, and for the split of
-// 512-row tiles, which callers size it by.
+// Workspace bytes of the plan of these sizes (0: no split, or no launch).
 inline int64_t plan_bytes(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll) {
-  const LaunchPlan best = plan_launch(m, tiles_o, nsteps, unroll, true);
-  if (best.kmt == 0) return 0;
-  const int64_t chosen = best.bytes;
-  const SplitPlan p = split_plan((m + tile_m(4) - 1) / tile_m(4) * tiles_o, nsteps, unroll,
-                                 launch_slots(4));
-  const int64_t whole = p.tail_tiles * p.splits * partial_floats(4) * (int64_t)sizeof(float);
-  return chosen > whole ? chosen : whole;
-}
-
-// The plan of a launch that has ws_bytes of workspace at ws.
-inline LaunchPlan plan_with(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll,
-                            const void *ws, int64_t ws_bytes) {
-  LaunchPlan p = plan_launch(m, tiles_o, nsteps, unroll, ws != nullptr);
-  if (p.split.tail_tiles > 0 && ws_bytes < p.bytes)
-    p = plan_launch(m, tiles_o, nsteps, unroll, false);
-  return p;
+  return plan_launch(m, tiles_o, nsteps, unroll, INT64_MAX).bytes;
 }
 
 // Fills in the launch's tiles and split; returns its work units, or -1 when

@@ -5,8 +5,8 @@ namespace nf4s {
 
 template <class Producer>
 static int32_t launch(GroupedArgs &ga, hipStream_t s, void *ws, int64_t ws_bytes) {
-  const LaunchPlan p =
-      plan_with(ga.base.M, ga.tiles_o, ga.base.R / kStep, Producer::kUnroll, ws, ws_bytes);
+  const LaunchPlan p = plan_launch(ga.base.M, ga.tiles_o, ga.base.R / kStep, Producer::kUnroll,
+                                   ws != nullptr ? ws_bytes : 0);
   const int64_t U = apply_plan(ga, p, ga.tiles_o, ws);
   if (U == 0) return NF4S_OK;
   if (U < 0) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");

@@ -5,7 +5,7 @@
 namespace nf4s {
 
 int32_t launch_swiglu(GroupedArgs &ga, bool dq, bool batch, hipStream_t s) {
-  const LaunchPlan p = plan_launch(ga.base.M, ga.tiles_o, ga.base.R / kStep, batch ? 4 : 2, false);
+  const LaunchPlan p = plan_launch(ga.base.M, ga.tiles_o, ga.base.R / kStep, batch ? 4 : 2, 0);
   const int64_t T = apply_plan(ga, p, ga.tiles_o, nullptr);
   if (T < 0) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
   with_kmt(p.kmt, [&](auto K) {

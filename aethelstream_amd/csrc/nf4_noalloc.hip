@@ -13,9 +13,11 @@
 
 namespace nf4s {
 
-// A split plan never needs more partial tiles than the device has CUs
-// (S <= CUs / r slices for r tail tiles), so 256 partial tiles (64 MiB)
-// cover every shape on a 256-CU MI355X.
+// A split plan never has more slices than the device runs workgroups at once:
+// one per CU with a partial of up to kGemmPartialTileBytes, or two per CU with
+// a quarter of it (128-row tiles); the few-token kernel's slices take at most
+// 32 or 64 KiB each.  256 of the largest (64 MiB) cover every shape on a
+// 256-CU MI355X.
 constexpr int64_t kScratchTiles = 256;
 constexpr int64_t kScratchBytes = kScratchTiles * kGemmPartialTileBytes;
 static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];

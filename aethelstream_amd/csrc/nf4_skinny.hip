@@ -440,7 +440,9 @@ static int sk_slices(int64_t tiles, int64_t steps, const SkShape &sh) {
   int64_t s = slots / tiles;
   const int64_t most = steps / (4 * sh.wk);  // at least 4 steps per wave
   if (s > most) s = most;
-  return (int)(s < 1 ? 1 : s);
+  if (s < 2) return 1;
+  const int64_t per = (steps + s - 1) / s;
+  return (int)((steps + per - 1) / per);  // slices of `per` steps that are not empty
 }
 
 static int64_t sk_tiles(int64_t n, int rows) { return (n + rows - 1) / rows; }
@@ -515,8 +517,9 @@ static int32_t sk_fwd_kind(const SkinnyArgs &all, bool dq, hipStream_t s, void *
   a.tiles = (int32_t)tiles;
   const int steps = (int)((a.k / 64 + 1) / 2);
   a.slices = sk_slices(tiles, steps, sh);
-  if (work == nullptr || work_bytes < a.slices * a.m * tiles * rows * (int64_t)sizeof(float))
-    a.slices = 1;
+  const int64_t per_slice = a.m * tiles * rows * (int64_t)sizeof(float);
+  const int64_t fit = work != nullptr ? work_bytes / per_slice : 0;
+  if (a.slices > fit) a.slices = fit < 2 ? 1 : (int)fit;
   a.slice_steps = (steps + a.slices - 1) / a.slices;
   a.slices = (steps + a.slice_steps - 1) / a.slice_steps;
   a.ws = static_cast<float *>(work);

@@ -50,8 +50,8 @@ struct SkinnyArgs {
 int64_t skinny_workspace_bytes(const int64_t *ns, int32_t count, int64_t m, int64_t k);
 
 // Runs the launch described by a (x, m, k, the groups' packed, am, out and
-// n); the plan (tiles, slices) is filled in here.  A NULL or too small
-// workspace runs without K slices.  0 < m <= kSkinnyMaxM.
+// n); the plan (tiles, slices) is filled in here: as many K slices as the
+// workspace holds, none with a NULL one.  0 < m <= kSkinnyMaxM.
 int32_t skinny_fwd(const SkinnyArgs &a, hipStream_t s, void *work, int64_t work_bytes);
 int32_t skinny_swiglu(SkinnyArgs &a, hipStream_t s);
 

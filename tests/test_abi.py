@@ -98,8 +98,9 @@ def test_dgrad_workspace_size_query():
     assert f(ns, 3, 256, 8192, None) == _lib.NF4S_ERR_INVALID_ARGUMENT
     assert f(ns, 0, 256, 8192, ctypes.byref(out)) == _lib.NF4S_ERR_INVALID_ARGUMENT
     assert f(ns, 5, 256, 8192, ctypes.byref(out)) == _lib.NF4S_ERR_INVALID_ARGUMENT
-    # 70B d_h1 at 256 tokens: 64 tiles -> 4 slices of 256 x 256 fp32 per thread.
-    assert f(ns, 3, 256, 8192, ctypes.byref(out)) == 0 and out.value == 64 * 4 * 256 * 256 * 4
+    # 70B d_h1 at 256 tokens: 64 tiles of 256 rows -> 4 slices of 256 threads x
+    # 128 fp32 partials each.
+    assert f(ns, 3, 256, 8192, ctypes.byref(out)) == 0 and out.value == 64 * 4 * 256 * 128 * 4
     # 8192 tokens: 1024 tiles, whole rounds, no split.
     assert f(ns, 3, 8192, 8192, ctypes.byref(out)) == 0 and out.value == 0
     # n % 64 != 0 is the GEMM's own error; the query reports no split.
@@ -146,6 +147,14 @@ def test_fwd_workspace_size_query():
     # 8192 x 8192 = 1024 tiles: whole rounds, no split.
     ns[0] = 8192
     assert f(ns, 1, 8192, 8192, ctypes.byref(out)) == 0 and out.value == 0
+    # 12800 columns at 512 tokens: the plan of least time (400 tiles of 256
+    # rows) has no split, so there is nothing to hold.
+    ns[0] = 12800
+    assert f(ns, 1, 512, 1024, ctypes.byref(out)) == 0 and out.value == 0
+    # 50 tokens of 5120 columns, K = 2304: 40 tiles of 128 columns in 2 slices
+    # of 9 steps, [slice][token][column] fp32.
+    ns[0] = 5120
+    assert f(ns, 1, 50, 2304, ctypes.byref(out)) == 0 and out.value == 2 * 50 * 5120 * 4
     # A negative workspace size is rejected before any launch.
     assert lib.nf4s_gemm_fwd_grouped_ws(0x1000, None, ns, None, 1, 64, 64, None, -1,
                                         None) == _lib.NF4S_ERR_INVALID_ARGUMENT

@@ -353,15 +353,28 @@ def test_swiglu_argument_errors():
 # would leave most CUs idle run as K slices; the fixup kernel sums their fp32
 # partials in slice order.  Only the fp32 summation order changes, so both the
 # split and the unsplit result stay within TOL_SAME of fp32 on the same
-# operands.  Shapes (on a 256-CU MI355X): T = 100 tiles -> 2 slices; 16 tiles
-# of ragged M and N -> 8 slices of 4 steps; the per-step producer with an odd
-# step count; a 7B gate/up pair (1376 tiles, the last 96 split in 2); 70B k
-# alone (128 tiles); a group mixing double-quant and fp32-absmax weights, which
-# runs one launch per kind over one workspace.
-SPLIT = [(512, [12800], 1024, True), (513, [1000], 2048, True), (512, [3840], 1344, False),
-         (512, [3840], 1344, True), (4096, [11008, 11008], 4096, True),
-         (8192, [1024], 8192, True), (700, [3000, 1200], 512, False),
-         (512, [6400, 1000, 6400], 1024, (True, False, False))]
+# operands.  Shapes (on a 256-CU MI355X): 64 tiles of 256 rows -> 4 slices of
+# 16 steps; 40 tiles of ragged M and N -> 8 slices of 4 steps; the per-step
+# producer with an odd step count; a 7B gate/up pair (1376 tiles, the last 96
+# split in 2); 70B k alone (128 tiles); a group mixing double-quant and
+# fp32-absmax weights, which runs one launch per kind over one workspace.
+# Every case runs on a workspace of a known pattern, of exactly the queried
+# size: partials in it show that the launch did split.
+PATTERN = 0xA5
+
+
+def _patterned(nbytes):
+    return torch.full((max(nbytes, 1),), PATTERN, dtype=torch.uint8, device=DEV)
+
+
+def _written(buf):
+    return bool((buf != PATTERN).any())
+
+
+SPLIT = [(512, [4096], 4096, True), (513, [1000], 2048, True), (512, [3840], 4160, False),
+         (512, [3840], 4160, True), (4096, [11008, 11008], 4096, True),
+         (8192, [1024], 8192, True), (700, [3000, 1200], 4096, False),
+         (512, [2048, 1000, 2048], 2048, (True, False, False))]
 
 
 @pytest.mark.parametrize("m,ns,k,dq", SPLIT)
@@ -371,9 +384,12 @@ def test_fwd_split_k_tail(m, ns, k, dq):
     dqs = dq if isinstance(dq, tuple) else (dq,) * len(ns)
     ws = [_weight(n, k, 61 + n + i, d) for i, (n, d) in enumerate(zip(ns, dqs))]
     x, xf = _act(m, k, 19 + m)
-    ys = gemm.linear_fwd_grouped(x, ws, split_k=True)
+    work = _patterned(need)
+    ys = gemm.linear_fwd_grouped(x, ws, split_k=True, workspace=work)
     ref = gemm.linear_fwd_grouped(x, ws, split_k=False)
     torch.cuda.synchronize()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert need > 0 and _written(work)  # these shapes do split on a 256-CU part
     for w, y, r in zip(ws, ys, ref):
         wdq = nf4.dequant(w).float()
         exact = x.float() @ wdq.t()
@@ -381,52 +397,86 @@ def test_fwd_split_k_tail(m, ns, k, dq):
         e_split = float((y.float() - exact).norm() / exact.norm())
         e_ref = float((r.float() - exact).norm() / exact.norm())
         assert e_split <= TOL_SAME and e_ref <= TOL_SAME, (e_split, e_ref)
-    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert need > 0  # these shapes do split on a 256-CU part
 
 
-def test_fwd_split_k_small_workspace_falls_back():
-    """A workspace smaller than one tile's partial sums, handed straight to the
-    C entry point (the Python wrapper would replace it): no split, the unsplit
-    result bit for bit."""
-    m, n, k = 512, 12800, 1024
-    w = _weight(n, k, 71, True)
-    x, _ = _act(m, k, 23)
-    small = torch.empty(4096, dtype=torch.uint8, device=DEV)
+def _fwd_on(x, w, work):
+    """linear_fwd with `work` handed straight to the C entry point (the Python
+    wrapper would replace a small one)."""
+    m, (n, k) = x.shape[0], w.shape
     y = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
     ns = (ctypes.c_int64 * 1)(n)
     ys = (ctypes.c_void_p * 1)(y.data_ptr())
     descs = (_lib.Nf4sTensor * 1)(w.descriptor())
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     _lib.check(_lib.load().nf4s_gemm_fwd_grouped_ws(x.data_ptr(), descs, ns, ys, 1, m, k,
-                                                    small.data_ptr(), 4096, stream))
-    r = gemm.linear_fwd(x, w, split_k=False)
+                                                    work.data_ptr(), work.numel(), stream))
     torch.cuda.synchronize()
-    assert torch.equal(y.view(torch.int16), r.view(torch.int16))
+    return y
+
+
+# The second shape is that of the few-token kernel, whose slices also go to
+# the workspace.
+@pytest.mark.parametrize("m,n,k", [(512, 4096, 4096), (50, 5120, 13824)])
+def test_fwd_split_k_small_workspace_falls_back(m, n, k):
+    """A workspace smaller than one tile's partial sums: no split, the unsplit
+    result bit for bit.  With the queried size the same call does split."""
+    w = _weight(n, k, 71, True)
+    x, _ = _act(m, k, 23)
+    print(f"small workspace m={m} n={n} k={k}", flush=True)
+    small, full = _patterned(4096), _patterned(gemm.fwd_workspace_bytes([n], m, k))
+    y = _fwd_on(x, w, small)
+    r = gemm.linear_fwd(x, w, split_k=False)
+    assert not _written(small) and torch.equal(y, r)
+    split = _fwd_on(x, w, full)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _written(full)
+    assert torch.equal(split, gemm.linear_fwd(x, w))
+
+
+@pytest.mark.parametrize("m,n,k,size", [(300, 4096, 8192, 40 << 20), (50, 5120, 13824, 10 << 20)])
+def test_fwd_split_k_takes_what_fits(m, n, k, size):
+    """A workspace too small for the best split still gets one that fits it
+    (other tile rows; fewer slices of the few-token kernel), and writes nothing
+    past its end."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the plans are those of a 256-CU part")
+    w = _weight(n, k, 75, True)
+    x, _ = _act(m, k, 25)
+    print(f"less workspace m={m} n={n} k={k}", flush=True)
+    assert gemm.fwd_workspace_bytes([n], m, k) > size
+    buf = _patterned(size + 4096)
+    y = _fwd_on(x, w, buf[:size])
+    assert _written(buf[:size]) and not _written(buf[size:])
+    exact = x.float() @ nf4.dequant(w).float().t()
+    assert float((y.float() - exact).norm() / exact.norm()) <= TOL_SAME
 
 
 def test_fwd_split_k_twice_in_a_row():
     """Two split launches on one stream reuse one workspace: the second (a
     smaller shape) must not see the first's partials."""
     ws_buf = torch.empty(64 << 20, dtype=torch.uint8, device=DEV)
-    for m, n, k, seed in ((512, 12800, 1024, 81), (256, 6400, 512, 82)):
+    for m, n, k, seed in ((512, 4096, 4096, 81), (256, 2048, 2048, 82)):
         w = _weight(n, k, seed, True)
         x, _ = _act(m, k, seed)
+        before = ws_buf.clone()
         y = gemm.linear_fwd_grouped(x, [w], split_k=True, workspace=ws_buf)[0]
         exact = x.float() @ nf4.dequant(w).float().t()
         torch.cuda.synchronize()
         assert float((y.float() - exact).norm() / exact.norm()) <= TOL_SAME
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert not torch.equal(before, ws_buf)  # both launches split
 
 
 
 # Split-K input gradient: few tokens leave a last round of at most half the
 # CUs, whose tiles then run as slices of the weights' concatenated reduction.
 # Cases: the batched producer (4 slices of 4 steps); the per-step producer
-# with a slice that straddles two summed weights (steps 10 + 5, slices of 4);
+# with a slice that straddles two summed weights (steps 10 + 5, slices of 4
+# or less);
 # the 70B d_h1 sum at 512 tokens (slices of 40 steps, the last one over the
 # end of Wq and all of Wk and Wv); two row blocks at ragged m.
 DGRAD_SPLIT = [(256, [1024], 1024, True), (300, [640, 320], 512, False),
-               (512, [8192, 1024, 1024], 8192, True), (1000, [2048], 4096, True)]
+               (512, [8192, 1024, 1024], 8192, True), (1000, [4096], 2048, True)]
 
 
 @pytest.mark.parametrize("m,ns,k,dq", DGRAD_SPLIT)
@@ -435,7 +485,8 @@ def test_dgrad_split_k_tail(m, ns, k, dq):
     ws = [_weight(n, k, 91 + n + i, dq) for i, n in enumerate(ns)]
     dys = [_act(m, n, 29 + n + i)[0] for i, n in enumerate(ns)]
     need = gemm.dgrad_workspace_bytes(ns, m, k)
-    got = gemm.linear_dgrad_sum(dys, ws, split_k=True)
+    work = _patterned(need)
+    got = gemm.linear_dgrad_sum(dys, ws, split_k=True, workspace=work)
     ref = gemm.linear_dgrad_sum(dys, ws, split_k=False)
     exact = sum(d.float() @ nf4.dequant(w).float() for d, w in zip(dys, ws))
     torch.cuda.synchronize()
@@ -443,7 +494,7 @@ def test_dgrad_split_k_tail(m, ns, k, dq):
     e_ref = float((ref.float() - exact).norm() / exact.norm())
     assert e_split <= TOL_SAME and e_ref <= TOL_SAME, (e_split, e_ref)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert need > 0  # these shapes do split on a 256-CU part
+        assert need > 0 and _written(work)  # these shapes do split on a 256-CU part
     if len(ns) == 1:
         one = gemm.linear_dgrad(dys[0], ws[0])
         torch.cuda.synchronize()
@@ -456,7 +507,7 @@ def test_dgrad_split_k_small_workspace_falls_back():
     m, n, k = 256, 1024, 1024
     w = _weight(n, k, 73, True)
     dy, _ = _act(m, n, 31)
-    small = torch.empty(4096, dtype=torch.uint8, device=DEV)
+    small = _patterned(4096)
     dx = torch.empty(m, k, dtype=torch.bfloat16, device=DEV)
     ns = (ctypes.c_int64 * 1)(n)
     dps = (ctypes.c_void_p * 1)(dy.data_ptr())
@@ -466,6 +517,7 @@ def test_dgrad_split_k_small_workspace_falls_back():
                                                   small.data_ptr(), 4096, stream))
     r = gemm.linear_dgrad(dy, w, split_k=False)
     torch.cuda.synchronize()
+    assert not _written(small)
     assert torch.equal(dx.view(torch.int16), r.view(torch.int16))
 
 
@@ -476,10 +528,13 @@ def test_dgrad_split_k_twice_in_a_row():
     for m, n, k, seed in ((512, 2048, 2048, 83), (256, 1024, 512, 84)):
         w = _weight(n, k, seed, True)
         dy, _ = _act(m, n, seed)
+        before = ws_buf.clone()
         dx = gemm.linear_dgrad(dy, w, split_k=True, workspace=ws_buf)
         exact = dy.float() @ nf4.dequant(w).float()
         torch.cuda.synchronize()
         assert float((dx.float() - exact).norm() / exact.norm()) <= TOL_SAME
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert not torch.equal(before, ws_buf)  # both launches split
 
 # Seeded random shapes: ragged m, any n for the forward (n % 64 == 0 for the
 # input gradient), k a multiple of 64 (per-step and batched producers), both

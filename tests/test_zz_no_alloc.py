@@ -57,8 +57,8 @@ def _run_pair(ws, m, k, seed):
 
 
 def test_noalloc_equals_workspace_entry_point_twice():
-    # Call 1: 8 output tiles on 256 CUs -> the largest split (64 MiB of
-    # partials at 32 slices).  Call 2: fewer tiles, rows and steps, a ragged
+    # Call 1: 32 tiles of 128 rows on 256 CUs, two workgroups a CU -> the most
+    # slices (32 MiB of partials at 16 slices).  Call 2: fewer tiles, rows and steps, a ragged
     # m, and a double-quant + fp32-absmax pair (two launches on the scratch).
     cases = [
         (_weights([(640, 8192, True), (384, 8192, True)], 1), 512, 8192),
