@@ -667,9 +667,14 @@ constexpr int kQuantU = 1;         // tiles per chunk
 constexpr int kQuantMaxGrid = 1024;  // workgroups of the quantize launches
 // Tiles per chunk with double-quant: 2 KB of x in flight per wave, one tile of
 // fp32 or two of bf16.  28672 x 8192 bf16 with one tile 114-119 us, two 109;
-// fp32 with one 200, two 204.
+// fp32 with one 200, two 204.  bf16 groups below 64 blocks have no two tiles
+// for each of the four waves: with chunks of two some waves idle, and a group
+// of one tile has no whole chunk and goes element by element (11008 x 4096,
+// group 8: 195 us with two, 130 with one; 16: 80 and 69; 32: 44.5 and 39.5;
+// 64: 26.9 and 27.5).
 template <typename T>
 constexpr int kQuantDqU = sizeof(T) == 4 ? 1 : 2;
+constexpr int32_t kQuantDqMinGroup = 64;
 
 template <typename T>
 static bool quantize_vec_ok(const T *x, const uint8_t *packed) {
@@ -709,12 +714,12 @@ static int32_t quantize_dq(const T *x, int64_t n, int32_t block_size, int32_t gr
   if (ng > 0x7fffffff) return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many groups");
   const size_t lds = (size_t)group * sizeof(float);
   const uint32_t grid = (uint32_t)(ng < kQuantMaxGrid ? ng : kQuantMaxGrid);
+  auto *kernel = quantize_dq_kernel<T, false, kQuantU>;
   if (quantize_vec_ok(x, packed))
-    hipLaunchKernelGGL((quantize_dq_kernel<T, true, kQuantDqU<T>>), dim3(grid), dim3(256), lds,
-                       as_stream(stream), x, n, group, packed, q, scale, nb, ng);
-  else
-    hipLaunchKernelGGL((quantize_dq_kernel<T, false, kQuantU>), dim3(grid), dim3(256), lds,
-                       as_stream(stream), x, n, group, packed, q, scale, nb, ng);
+    kernel = group < kQuantDqMinGroup ? quantize_dq_kernel<T, true, 1>
+                                      : quantize_dq_kernel<T, true, kQuantDqU<T>>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, as_stream(stream), x, n, group, packed, q,
+                     scale, nb, ng);
   return check_launch("quantize_dq_kernel");
 }
 

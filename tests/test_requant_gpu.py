@@ -58,6 +58,22 @@ def test_quantize_dq_fused_vs_oracle(n, group, bf16):
 
 
 
+# bf16 groups on both sides of the line between one and two tiles (8 blocks) a
+# step: a whole tile, a tile short of a step, and a partial last group.
+@pytest.mark.parametrize("group", [8, 16, 32, 64, 128])
+def test_quantize_dq_bf16_group_sizes(group):
+    n = 64 * group * 5 + 64 * 9 + 33
+    print(f"quantize_dq group={group} n={n}", flush=True)
+    t, ref_in = _values(n, 300 + group, True)
+    w = nf4.quantize_weight(t, double_quant=True, dq_group=group)
+    pk_ref, am_ref = oracle.quantize_nf4(ref_in)
+    q_ref, s_ref = oracle.dq_encode(am_ref, group)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(w.packed.cpu().numpy(), pk_ref)
+    np.testing.assert_array_equal(w.absmax_q.cpu().numpy(), q_ref)
+    np.testing.assert_array_equal(_u32(w.absmax_scale), s_ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("group,bf16", [(8, False), (16, True), (256, False)])
 def test_quantize_dq_more_groups_than_workgroups(group, bf16):
     # The fused kernel's workgroups each take several groups in turn once
