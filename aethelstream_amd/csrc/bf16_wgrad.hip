@@ -241,8 +241,8 @@ __device__ __forceinline__ void wgrad_close_step(int64_t t, int64_t nsteps) {
   });
 }
 
-// Direct epilogue, for ragged columns and outputs without 16-byte stores: four
-// adjacent fp32 per store.
+// Direct epilogue, for outputs without 16-byte stores: four adjacent fp32 per
+// store or less.
 template <bool kAcc, int kMT>
 __device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[kMT][4], float *dw,
                                          int64_t n0, int64_t k0, int64_t N, int lane,
@@ -275,20 +275,26 @@ __device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&ac
   }
 }
 
-// Epilogue through LDS for whole-width tiles: the direct stores write 32 rows
-// x 32 bytes per instruction, these two whole 512-byte rows.  Per 32-row block
-// mt the wave writes its 32 x 128 fp32 to its own 16 KB of the idle ring (row
-// r, 16-byte chunk c at physical chunk c ^ r: the lanes of a ds_write_b128
-// share c, those of a ds_read_b128 r, both spread over all banks), reads it
-// back by rows and stores; to accumulate, 8 of dW's old row pairs are loaded
-// at a time.  The tile's output burst (64 MB a round over the chip) is what a
-// short reduction waits for: against the direct stores, same box, 2 x 11008 x
-// 4096 over 1000 tokens 245 -> 231 us (326 -> 273 accumulating), 28672 x 8192
-// over 512 tokens 384 -> 319 (600 -> 484), 8192 x 8192 over 8192 tokens 846 ->
-// 826 (909 -> 867).  Non-temporal stores: without them 367 us for 28672 x 8192
-// over 512 tokens.  Accumulating is its own instantiation: as a run-time test
-// it spilled 51 registers in both.
-template <bool kAcc, int kMT>
+// Epilogue through LDS for outputs that take 16-byte stores: the direct stores
+// write 32 rows x 32 bytes per instruction, these two whole 512-byte rows.
+// Per 32-row block mt the wave writes its 32 x 128 fp32 to its own 16 KB of
+// the idle ring (row r, 16-byte chunk c at physical chunk c ^ r: the lanes of a
+// ds_write_b128 share c, those of a ds_read_b128 r, both spread over all
+// banks), reads it back by rows and stores; to accumulate, 8 of dW's old row
+// pairs are loaded at a time.  Chunks past the last column are dropped: K is a
+// multiple of 8, so none is partial.  (Direct stores for the tiles of a ragged
+// last column, all on the XCD that takes the last strip, kept it busy after
+// the others: 15696 x 6120 over 100 tokens 118 -> 94 us, accumulating 270 ->
+// 165.)
+// The tile's output burst (64 MB a round over the chip) is what a short
+// reduction waits for: against the direct stores, same box, 2 x 11008 x 4096
+// over 1000 tokens 245 -> 231 us (326 -> 273 accumulating), 28672 x 8192 over
+// 512 tokens 384 -> 319 (600 -> 484), 8192 x 8192 over 8192 tokens 846 -> 826
+// (909 -> 867).
+// kNt: non-temporal stores (wg_nontemporal).  Accumulating and the store policy
+// are instantiations: as a run-time test accumulating spilled 51 registers in
+// both, the policy 9.
+template <bool kAcc, int kMT, bool kNt>
 __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 (&acc)[kMT][4],
                                              floatx4 *lds, float *dw, int64_t n0, int64_t k0,
                                              int64_t N, int lane) {
@@ -299,13 +305,15 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
   const int r0 = lane >> 5, c = lane & 31;  // read-back: row 2i + r0, chunk c
   // The wave's rows below N through a buffer resource that ends after the last.
   const int64_t left = N - n0;
-  const int64_t rows = left <= 0 ? 0 : (left > 32 * kMT ? 32 * kMT : left);
+  const int64_t cols = g.K - k0;  // <= 0 for a wave past the last column
+  const int64_t rows = left <= 0 || cols <= 0 ? 0 : (left > 32 * kMT ? 32 * kMT : left);
   const uint32_t ld4 = (uint32_t)(g.K * 4);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
       (void *)(rows > 0 ? dw + n0 * g.K + k0 : dw), 0,
-      rows > 0 ? (int32_t)((rows - 1) * ld4 + 512) : 0, kBufferFlags);
+      rows > 0 ? (int32_t)((rows - 1) * ld4 + 4 * (uint32_t)(cols < 128 ? cols : 128)) : 0,
+      kBufferFlags);
   typedef unsigned int uvec4 __attribute__((ext_vector_type(4)));
-  constexpr int kStoreNt = 2;  // non-temporal
+  constexpr int kPolicy = kNt ? 2 : 0;
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt) {
     const uint32_t base = (uint32_t)(32 * mt + r0) * ld4 + 16u * (uint32_t)c;
@@ -323,6 +331,7 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int h = 0; h < 16; h += 8) {
+      if (4 * c >= cols) continue;  // a lane past the last column
       floatx4 v[8], old[8];
       if constexpr (kAcc) {
 #pragma unroll
@@ -341,7 +350,7 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
         if constexpr (kAcc) v[i] += old[i];
         __builtin_amdgcn_raw_buffer_store_b128(
             __builtin_bit_cast(uvec4, v[i]), rs,
-            (int)(base + 2u * (uint32_t)(h + i) * ld4), 0, kStoreNt);
+            (int)(base + 2u * (uint32_t)(h + i) * ld4), 0, kPolicy);
       }
     }
     asm volatile("" ::: "memory");
@@ -351,7 +360,7 @@ __device__ __forceinline__ void wg_store_lds(const WgradArgs &g, const floatx16 
 }
 
 // One output tile: its 64 kMT x 256 dW block over all M tokens.
-template <bool kAcc, int kMT>
+template <bool kAcc, int kMT, bool kNt>
 __global__ void __launch_bounds__(kWgThreads, 4 / kMT) wgrad_kernel(const WgradArgs g) {
   const int T = g.tiles_n * g.tiles_k;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -481,8 +490,9 @@ __global__ void __launch_bounds__(kWgThreads, 4 / kMT) wgrad_kernel(const WgradA
     // columns k = k0 + 128 hk + 32 nt + 8 j + 4 (l / 32) + i in registers
     // 4 j + i of tile [mt][nt].
     const bool vec_ok = ((reinterpret_cast<uintptr_t>(dw) & 15) == 0) && ((g.K & 3) == 0);
-    if (vec_ok && k0 + kWgTile <= g.K && g.K < ((int64_t)1 << 22))  // 32-bit row offsets
-      wg_store_lds<kAcc, kMT>(g, acc, lds_wave, dw, n0 + 32 * kMT * hn, k0 + 128 * hk, N, lane);
+    if (vec_ok && g.K < ((int64_t)1 << 22))  // 32-bit row offsets
+      wg_store_lds<kAcc, kMT, kNt>(g, acc, lds_wave, dw, n0 + 32 * kMT * hn, k0 + 128 * hk, N,
+                                   lane);
     else
       wg_store<kAcc, kMT>(g, acc, dw, n0 + 32 * kMT * hn, k0 + 128 * hk, N, lane, vec_ok);
     // The next tile's prologue DMAs overwrite the LDS that the last step and
@@ -523,6 +533,26 @@ static int wg_tile_mt(const int64_t *ns, int32_t count, int64_t m, int64_t tiles
                        (rest == 0 ? 0.0 : (rest <= cus ? 0.65 : full));
   const double cost4 = (double)((tiles4 * tiles_k + cus - 1) / cus);
   return cost2 < cost4 ? 2 : 4;
+}
+
+// Whether dW (not accumulated) is stored non-temporally: 28672 x 8192 over 512
+// tokens 319 us with, 367 without.  Rows that are no multiple of 128 bytes
+// share their first and last cache lines with their neighbours, and only a
+// cache merges the two parts.  So they keep the default policy while the stores
+// set the time and dW (nearly) fits in the Infinity Cache of 256 MB (times with
+// / without non-temporal stores, us):
+//   16000 x 4104 (250 MiB), 16 tokens 69 / 45, 128 67 / 52, 1024 150 / 146,
+//   3000 355 / 357, 4096 474 / 501;
+//   24000 x 4104 (376 MiB), 128 tokens 97 / 89, 256 101 / 110, 1024 219 / 241.
+// A larger dW of very few tokens keeps it too, unless whole 64-byte halves of
+// the lines are written (28672 x 5000, 128 tokens 166 / 145; 28672 x 8208, a
+// multiple of 16, 171 / 203).
+constexpr int64_t kWgFewTokens = 160;
+static bool wg_nontemporal(const int64_t *ns, int32_t count, int64_t m, int64_t k) {
+  if (k % 32 == 0 || m > 3072) return true;
+  int64_t bytes = 0;
+  for (int i = 0; i < count; ++i) bytes += 4 * ns[i] * k;
+  return bytes > ((int64_t)288 << 20) && (k % 16 == 0 || m > kWgFewTokens);
 }
 
 static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, float *const *dws,
@@ -627,7 +657,12 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
   // stores (28672 x 8192 over 256 tokens: 188 us with 8, 203 with 4; 2 x 11008
   // x 4096 over 1000: 181 and 176, over 8192: 1289 and 1232).
   g.strip = (mt == 2 && m > 512) ? 4 : 8;
-  if (g.strip > g.tiles_k) g.strip = g.tiles_k;
+  // Stores of the default policy meet their neighbours' halves of a line in the
+  // cache if whole rows of dW are under way at once: with so few tokens that
+  // the operands hardly count, the strip is the whole width (16000 x 10808
+  // over 81 tokens 181 -> 168 us, 32840 x 12072 439 -> 400).
+  const bool nt = accumulate || wg_nontemporal(ns, count, m, k);
+  if (g.strip > g.tiles_k || (!nt && m <= kWgFewTokens)) g.strip = g.tiles_k;
   if (G % 8 == 0 && T % G == 0) {
     const int S = (int)(G / 8);
     int best = 0;
@@ -642,8 +677,11 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
       }
     }
   }
-  auto *kernel = mt == 4 ? (accumulate ? wgrad_kernel<true, 4> : wgrad_kernel<false, 4>)
-                         : (accumulate ? wgrad_kernel<true, 2> : wgrad_kernel<false, 2>);
+  auto *kernel = mt == 4 ? wgrad_kernel<true, 4, true> : wgrad_kernel<true, 2, true>;
+  if (!accumulate && nt)
+    kernel = mt == 4 ? wgrad_kernel<false, 4, true> : wgrad_kernel<false, 2, true>;
+  else if (!accumulate)
+    kernel = mt == 4 ? wgrad_kernel<false, 4, false> : wgrad_kernel<false, 2, false>;
   hipLaunchKernelGGL(kernel, dim3((uint32_t)G), dim3(kWgThreads), 0, s, g);
   return check_launch("wgrad_kernel");
 }
