@@ -19,6 +19,8 @@
 // tokens, and than 4 or 5 of 32), and each wave reads its fragments with
 // the transposing ds_read_b64_tr_b16: 8 consecutive tokens of one column
 // per lane.
+#include <cmath>
+
 #include "abi_common.hpp"
 #include "gemm_common.hpp"
 #include "nf4_device.hpp"
@@ -511,27 +513,43 @@ __global__ void fill_zero_f32(float *__restrict__ p, int64_t n) {
 // tiles, two workgroups a CU).  Two workgroups hide one's stores and first
 // loads behind the other's products, and half tiles leave less of a last round
 // idle; but each x fragment feeds half the products.  The costs below are in
-// rounds of 256-row tiles, one per CU.  A full round of 128-row tiles (two a
-// CU) against it, 8192 x 8192: 256 tokens 57 us against 76, 1000 tokens 130
-// against 146, 2048 tokens 234 against 242, 4096 tokens 432 against 421, 8192
-// tokens 850 against 808; a round with one 128-row tile a CU takes 0.58-0.7.
-// 6000 x 3000 (1.1 rounds against 2) over 4096 tokens: 156 against 189 us;
-// 1024 x 8192 over 1000 tokens: 23 against 31; 1024 x 1024 over 1000: 15
-// against 25.
+// full rounds of 256-row tiles, fitted to 852 shapes (16 to 8192 tokens, 512 to
+// 56000 rows, 1024 to 16384 columns, a tenth of a round to 27): the choice
+// takes 0.4 % more time than the better of the two on average.
+// One round of 128-row tiles (two a CU) takes 0.78 at 256 tokens and 0.055 more
+// with each doubling, in a row of rounds 0.84 and 0.045 (8192 x 8192: 256
+// tokens 57 us against 76, 1000 tokens 130 against 146, 2048 tokens 234 against
+// 242, 4096 tokens 432 against 421, 8192 tokens 850 against 808).  Once the
+// operands come near the Infinity Cache's 256 MB, dy comes from memory in rows
+// of 256 bytes: up to 1.3 times that (27176 x 2528 over 8000 tokens 1138 us
+// against 977, 39848 x 7184 over 6783 tokens 1.45 times).
+// A round that fills a share f of the chip is no full one, its workgroups run
+// faster: 0.62 to 0.70 up to half the chip and in proportion beyond; with
+// 128-row tiles 0.4 to 0.6, then 0.75 as soon as a CU has two (0.82 after whole
+// rounds, whose ends are not in step).
 // tiles4: 256-row tile rows of all products.  Called on sizes whose tile count
 // fits 31 bits (a 128-row tiling that would not keeps the 256-row one).
-static int wg_tile_mt(const int64_t *ns, int32_t count, int64_t m, int64_t tiles4,
+static int wg_tile_mt(const int64_t *ns, int32_t count, int64_t m, int64_t k, int64_t tiles4,
                       int64_t tiles_k) {
   const int64_t cus = cu_slots();
   int64_t tiles2 = 0;
   for (int i = 0; i < count; ++i) tiles2 += (ns[i] + 127) / 128;
   if (tiles2 * tiles_k > 0x7fffffff) return 4;
   const int64_t t2 = tiles2 * tiles_k;
-  const double full = m <= 1024 ? 0.95 : (m <= 2048 ? 1.0 : 1.06);
-  const int64_t rest = t2 % (2 * cus);
-  const double cost2 = (double)(t2 / (2 * cus)) * full +
-                       (rest == 0 ? 0.0 : (rest <= cus ? 0.65 : full));
-  const double cost4 = (double)((tiles4 * tiles_k + cus - 1) / cus);
+  double n = (double)k;
+  for (int i = 0; i < count; ++i) n += (double)ns[i];
+  const double doublings = std::log2((double)(m < 128 ? 128 : m)) - 8.0;
+  const double past = (2e-6 * n * (double)m - 220.0) / 450.0;  // MB of dy and x
+  const double far = past < 0.0 ? 1.0 : (past > 0.3 ? 1.3 : 1.0 + past);
+  const int64_t t4 = tiles4 * tiles_k;
+  const double f2 = (double)(t2 % (2 * cus)) / (double)(2 * cus);
+  const double f4 = (double)(t4 % cus) / (double)cus;
+  const double two = t2 < 2 * cus ? 0.50 : 0.57;
+  const double part2 = f2 == 0.0 ? 0.0 : (f2 <= 0.5 ? 0.40 + 0.4 * f2 : two + 0.5 * f2);
+  const double part4 = f4 == 0.0 ? 0.0 : (f4 <= 0.5 ? 0.62 + 0.16 * f4 : 0.40 + 0.6 * f4);
+  const double cost2 = far * ((0.84 + 0.045 * doublings) * (double)(t2 / (2 * cus)) +
+                              (0.78 + 0.055 * doublings) * part2);
+  const double cost4 = (double)(t4 / cus) + part4;
   return cost2 < cost4 ? 2 : 4;
 }
 
@@ -623,7 +641,7 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
   }
   if (tiles_n * g.tiles_k > 0x7fffffff)
     return fail(NF4S_ERR_UNSUPPORTED_SHAPE, "too many tiles");
-  const int mt = wg_tile_mt(ns, count, m, tiles_n, g.tiles_k);
+  const int mt = wg_tile_mt(ns, count, m, k, tiles_n, g.tiles_k);
   tiles_n = 0;
   for (int i = 0; i < count; ++i) {
     g.tile0[i] = (int32_t)tiles_n;
@@ -647,30 +665,35 @@ static int32_t wgrad_grouped(const uint16_t *const *dys, const int64_t *ns, floa
     }
     return NF4S_OK;
   }
-  // XCD blocks (wg_map_tile) when every round is full: the squarest
-  // blk_n x blk_k = G / 8 that divides the tile grid (the products' tile
-  // rows stacked).
   const int64_t slots = (int64_t)cu_slots() * (4 / mt);
   const int64_t G = T < slots ? T : slots;
-  // Strips of 8 tile columns; the 64 slots of an XCD with 128-row tiles read
-  // less per step from strips of 4, which pays once the steps outweigh the
-  // stores (28672 x 8192 over 256 tokens: 188 us with 8, 203 with 4; 2 x 11008
-  // x 4096 over 1000: 181 and 176, over 8192: 1289 and 1232).
-  g.strip = (mt == 2 && m > 512) ? 4 : 8;
+  // Strips of about 8 tile columns; the 64 slots of an XCD with 128-row tiles
+  // read less per step from strips of about 4, which pays once the steps
+  // outweigh the stores (28672 x 8192 over 256 tokens: 188 us with 8, 203 with
+  // 4; 2 x 11008 x 4096 over 1000: 181 and 176, over 8192: 1289 and 1232).  All
+  // of one width: a last strip of one column reads all of dy for it (56000 x
+  // 1080 over 2841 tokens, 4 + 1 columns 446 us, 5 412).
+  const int want = (mt == 2 && m > 512) ? 4 : 8;
+  const int strips = g.tiles_k < want ? 1 : (g.tiles_k + want / 2) / want;
+  g.strip = (g.tiles_k + strips - 1) / strips;
   // Stores of the default policy meet their neighbours' halves of a line in the
   // cache if whole rows of dW are under way at once: with so few tokens that
   // the operands hardly count, the strip is the whole width (16000 x 10808
   // over 81 tokens 181 -> 168 us, 32840 x 12072 439 -> 400).
   const bool nt = accumulate || wg_nontemporal(ns, count, m, k);
-  if (g.strip > g.tiles_k || (!nt && m <= kWgFewTokens)) g.strip = g.tiles_k;
-  if (G % 8 == 0 && T % G == 0) {
-    const int S = (int)(G / 8);
-    int best = 0;
+  if (!nt && m <= kWgFewTokens) g.strip = g.tiles_k;
+  // XCD blocks (wg_map_tile) when every round is full: the squarest
+  // blk_n x blk_k = G / 8 that divides the tile grid (the products' tile
+  // rows stacked), if an XCD then reads no more per step than with strips (59
+  // x 8 tiles only divide into 59 x 1, which reads all of dy on every XCD).
+  if (G % 8 == 0 && T % G == 0 && (nt || m > kWgFewTokens)) {
+    const int S = (int)(G / 8), w = g.strip < S ? g.strip : S;
+    int best = mt * ((S + w - 1) / w) + 4 * w;  // columns read per XCD and step, in 64s
     for (int bn = 1; bn <= S; ++bn) {
       if (S % bn != 0 || g.tiles_n % bn != 0 || g.tiles_k % (S / bn) != 0) continue;
       const int bk = S / bn;
-      const int cost = mt * bn + 4 * bk;  // columns read per XCD and step, in 64s
-      if (best == 0 || cost < best) {
+      const int cost = mt * bn + 4 * bk;
+      if (cost < best || (cost == best && g.blk_n == 0)) {
         best = cost;
         g.blk_n = bn;
         g.blk_k = bk;
