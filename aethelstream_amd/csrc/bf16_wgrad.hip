@@ -176,7 +176,8 @@ __device__ __forceinline__ void wgrad_step(floatx16 (&acc)[kMT][4], u32x4 (&fd)[
                                            const char *__restrict__ cur_x,
                                            char *__restrict__ nxt_dy, char *__restrict__ nxt_x,
                                            const uint32_t (&rdy)[kMT], const uint32_t (&rx)[4],
-                                           __amdgpu_buffer_rsrc_t rs_dy, __amdgpu_buffer_rsrc_t rs_x,
+                                           __amdgpu_buffer_rsrc_t rs_dy,
+                                           __amdgpu_buffer_rsrc_t rs_x,
                                            uint32_t (&vdy)[kMT], uint32_t (&vx)[4],
                                            uint32_t step_dy, uint32_t step_x, bool more, int wave) {
   constexpr int kReads = kMT + 4, kDmas = kMT + 4;
@@ -246,8 +247,8 @@ __device__ __forceinline__ void wgrad_close_step(int64_t t, int64_t nsteps) {
 // Direct epilogue, for outputs without 16-byte stores: four adjacent fp32 per
 // store or less.
 template <bool kAcc, int kMT>
-__device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[kMT][4], float *dw,
-                                         int64_t n0, int64_t k0, int64_t N, int lane,
+__device__ __forceinline__ void wg_store(const WgradArgs &g, const floatx16 (&acc)[kMT][4],
+                                         float *dw, int64_t n0, int64_t k0, int64_t N, int lane,
                                          bool vec_ok) {
   asm volatile("" : "+v"(lane));  // as in wg_store_lds
   const int jl = lane & 31, grp = lane >> 5;
@@ -466,7 +467,7 @@ __global__ void __launch_bounds__(kWgThreads, 4 / kMT) wgrad_kernel(const WgradA
         constexpr int i = decltype(I)::value;
         constexpr int c = i, nx = (i + kWgStages - 1) % kWgStages;
         wgrad_step<kMT>(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
-                   step_dy, step_x, t + i + kWgStages - 1 < nsteps, wave);
+                        step_dy, step_x, t + i + kWgStages - 1 < nsteps, wave);
         wgrad_close_step<kMT>(t + i, nsteps);
       });
     }
@@ -475,7 +476,7 @@ __global__ void __launch_bounds__(kWgThreads, 4 / kMT) wgrad_kernel(const WgradA
       constexpr int c = i, nx = (i + kWgStages - 1) % kWgStages;
       if (t + i < nsteps) {
         wgrad_step<kMT>(acc, fd, fx, ldy[c], lx[c], ldy[nx], lx[nx], rdy, rx, rs_dy, rs_x, vdy, vx,
-                   step_dy, step_x, false, wave);
+                        step_dy, step_x, false, wave);
         wgrad_close_step<kMT>(t + i, nsteps);
       }
     });

@@ -1,6 +1,6 @@
 // gemm_common.hpp - pieces shared by the MFMA GEMM kernels for gfx950: vector
 // types, compile-time loops, s_waitcnt encodings, the step barrier, the
-// XCD-aware tile order and the persistent grid size.
+// XCD-aware tile order and the compute-unit count.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -85,12 +85,9 @@ __device__ __forceinline__ void map_tile(int b, int tiles_m, int tiles_o, int &t
   to = L - tm * tiles_o;
 }
 
-// Persistent grid: one workgroup per compute unit (a workgroup takes all or
-// most of a CU's LDS), each looping over tiles b, b + grid, ...  A tile's
-// output stores then drain while the same workgroup's next tile starts
-// loading.  The CU count is read once per device; a multiple of 8 keeps tile
-// b on XCD b % 8 (map_tile).
-// The current device's compute-unit count rounded up to a multiple of 8.
+// The current device's compute-unit count rounded up to a multiple of 8, which
+// keeps tile b of a persistent grid of that size (or twice it) on XCD b % 8
+// (map_tile).  Read once per device.
 inline int cu_slots() {
   static std::atomic<int> cus[64];  // zero-initialized (static storage)
   int dev = 0;
@@ -105,11 +102,6 @@ inline int cu_slots() {
     cus[dev].store(c, std::memory_order_relaxed);  // every caller stores the same value
   }
   return c;
-}
-
-inline uint32_t persistent_grid(int64_t tiles) {
-  const int c = cu_slots();
-  return (uint32_t)(tiles < c ? tiles : c);
 }
 
 }  // namespace nf4s

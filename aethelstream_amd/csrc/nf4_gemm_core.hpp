@@ -792,8 +792,9 @@ __device__ __forceinline__ void gemm_step(const GemmArgs &g, Producer &prod,
                                           floatx16 (&acc)[kMT][4], u32x4 (&a)[2][kMT],
                                           u32x4 (&b)[2][4], u32x4 *Acur, u32x4 *Aoth,
                                           const u32x4 *Bcur, u32x4 *Bnext,
-                                          __amdgpu_buffer_rsrc_t arsrc, const uint32_t (&aoff)[4 * kMT],
-                                          int t, int nsteps, int jl, int grp) {
+                                          __amdgpu_buffer_rsrc_t arsrc,
+                                          const uint32_t (&aoff)[4 * kMT], int t, int nsteps,
+                                          int jl, int grp) {
   constexpr int kPar = 1 - (kPhase & 1);
   constexpr const char *plan = SlotPlan<kMT>::plan;
   constexpr int kSub = 4 * kMT;     // MFMAs of a sub-step
@@ -835,62 +836,62 @@ __device__ __forceinline__ void gemm_step(const GemmArgs &g, Producer &prod,
         __builtin_bit_cast(bf16x8, b[s & 1][nt]), __builtin_bit_cast(bf16x8, a[s & 1][mt]),
         acc[mt][nt], 0, 0, 0);
     static_for<plan_slot(plan, n), plan_slot(plan, n + 1) - 1>([&](auto P) {
-    constexpr int pos = decltype(P)::value;
-    constexpr char kind = plan[pos];
-    if constexpr (kind == 'r') {
-      constexpr int q = plan_index(plan, pos, 'r');
-      constexpr int rs = 1 + q / kReads;
-      read_frag<kMT>(prod, Acur, Bcur, a, b, rs, q % kReads, rs & 1, jl, grp);
-    }
-    if constexpr (kind == 'N') dma(Aoth, 2 * kMT + plan_index(plan, pos, 'N'), t1);
-    if constexpr (kind == 'A') {
-      constexpr int d = plan_index(plan, pos, 'A');
-      // The wave's reads of Acur (sub-step 3's fragments) have returned;
-      // weight-tile stores issued after them may still be pending.
-      if constexpr (d == 0)
-        __builtin_amdgcn_s_waitcnt(kWaitLgkm0 | (stores_after_reads(plan, pos) << 8));
-      dma(Acur, d, t2);
-    }
-    if constexpr (kind == 'M') {
-      // Entries 2j and 2j+1 of this lane's half of the table.
-      constexpr int j = plan_index(plan, pos, 'M');
-      const float p0 = fp32_rounded(prod.code[2 * j] * ta);
-      const float p1 = fp32_rounded(prod.code[2 * j + 1] * ta);
-      lutd[j & 1] = pack_bf16x2(p0, p1);
-      if constexpr (j & 1) {
-        own[2 * (j >> 1)] = perm(lutd[1], lutd[0], 0x06040200u);
-        own[2 * (j >> 1) + 1] = perm(lutd[1], lutd[0], 0x07050301u);
+      constexpr int pos = decltype(P)::value;
+      constexpr char kind = plan[pos];
+      if constexpr (kind == 'r') {
+        constexpr int q = plan_index(plan, pos, 'r');
+        constexpr int rs = 1 + q / kReads;
+        read_frag<kMT>(prod, Acur, Bcur, a, b, rs, q % kReads, rs & 1, jl, grp);
       }
-    }
-    if constexpr (kind == 'D') {
-      // (own half, partner's half): see HalfTable.
-      static_for<0, 2>([&](auto Q) {
-        constexpr int q = decltype(Q)::value;
-        lut.lo[q] = own[2 * q];
-        lut.hi[q] = own[2 * q + 1];
-        lut.lo[2 + q] = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[2 * q], Producer::kDppPartner,
-                                                           0xf, 0xf, false);
-        lut.hi[2 + q] = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[2 * q + 1],
-                                                           Producer::kDppPartner, 0xf, 0xf, false);
-      });
-    }
-    if constexpr (kind == 'W') {
-      constexpr int j = plan_index(plan, pos, 'W');
-      constexpr int k = j / kWordStages, stage = j % kWordStages;
-      if constexpr (stage == 0) {
-        nat_select(prod.template word<kPhase>(k) ^ prod.hmask, wl);
-      } else if constexpr (stage == 1) {
-        nat_controls(wl);
-      } else if constexpr (stage == 2) {
-        nat_planes_a(lut, wl);
-      } else if constexpr (stage == 3) {
-        nat_planes_b(lut, wl);
-      } else if constexpr (stage == 4) {
-        nat_merge(wl, wp[k]);
-      } else {
-        prod.template store<kPar, k, 0>(Bnext, wp[k]);
+      if constexpr (kind == 'N') dma(Aoth, 2 * kMT + plan_index(plan, pos, 'N'), t1);
+      if constexpr (kind == 'A') {
+        constexpr int d = plan_index(plan, pos, 'A');
+        // The wave's reads of Acur (sub-step 3's fragments) have returned;
+        // weight-tile stores issued after them may still be pending.
+        if constexpr (d == 0)
+          __builtin_amdgcn_s_waitcnt(kWaitLgkm0 | (stores_after_reads(plan, pos) << 8));
+        dma(Acur, d, t2);
       }
-    }
+      if constexpr (kind == 'M') {
+        // Entries 2j and 2j+1 of this lane's half of the table.
+        constexpr int j = plan_index(plan, pos, 'M');
+        const float p0 = fp32_rounded(prod.code[2 * j] * ta);
+        const float p1 = fp32_rounded(prod.code[2 * j + 1] * ta);
+        lutd[j & 1] = pack_bf16x2(p0, p1);
+        if constexpr (j & 1) {
+          own[2 * (j >> 1)] = perm(lutd[1], lutd[0], 0x06040200u);
+          own[2 * (j >> 1) + 1] = perm(lutd[1], lutd[0], 0x07050301u);
+        }
+      }
+      if constexpr (kind == 'D') {
+        // (own half, partner's half): see HalfTable.
+        static_for<0, 2>([&](auto Q) {
+          constexpr int q = decltype(Q)::value;
+          lut.lo[q] = own[2 * q];
+          lut.hi[q] = own[2 * q + 1];
+          lut.lo[2 + q] = (uint32_t)__builtin_amdgcn_mov_dpp(
+              (int)own[2 * q], Producer::kDppPartner, 0xf, 0xf, false);
+          lut.hi[2 + q] = (uint32_t)__builtin_amdgcn_mov_dpp(
+              (int)own[2 * q + 1], Producer::kDppPartner, 0xf, 0xf, false);
+        });
+      }
+      if constexpr (kind == 'W') {
+        constexpr int j = plan_index(plan, pos, 'W');
+        constexpr int k = j / kWordStages, stage = j % kWordStages;
+        if constexpr (stage == 0) {
+          nat_select(prod.template word<kPhase>(k) ^ prod.hmask, wl);
+        } else if constexpr (stage == 1) {
+          nat_controls(wl);
+        } else if constexpr (stage == 2) {
+          nat_planes_a(lut, wl);
+        } else if constexpr (stage == 3) {
+          nat_planes_b(lut, wl);
+        } else if constexpr (stage == 4) {
+          nat_merge(wl, wp[k]);
+        } else {
+          prod.template store<kPar, k, 0>(Bnext, wp[k]);
+        }
+      }
     });
     __builtin_amdgcn_sched_barrier(0);
   });
@@ -964,17 +965,17 @@ __device__ __forceinline__ void gemm_main(const GemmArgs &g, Producer &prod,
     static_for<0, U>([&](auto P) {
       constexpr int p = decltype(P)::value;
       if constexpr ((p & 1) == 0)
-        gemm_step<kMT, Producer, p>(g, prod, acc, fa, fb, A0, A1, B0, B1, arsrc, aoff, t + p, nsteps,
-                               jl, grp);
+        gemm_step<kMT, Producer, p>(g, prod, acc, fa, fb, A0, A1, B0, B1, arsrc, aoff, t + p,
+                                    nsteps, jl, grp);
       else
-        gemm_step<kMT, Producer, p>(g, prod, acc, fa, fb, A1, A0, B1, B0, arsrc, aoff, t + p, nsteps,
-                               jl, grp);
+        gemm_step<kMT, Producer, p>(g, prod, acc, fa, fb, A1, A0, B1, B0, arsrc, aoff, t + p,
+                                    nsteps, jl, grp);
     });
   }
   if constexpr (U == 2) {
     if (t < nsteps)
       gemm_step<kMT, Producer, 0>(g, prod, acc, fa, fb, A0, A1, B0, B1, arsrc, aoff, t, nsteps, jl,
-                             grp);
+                                  grp);
   }
   gemm_tail<kMT>(acc, fa, fb);
   // No LDS DMA may still be in flight when the workgroup's LDS is released.
@@ -1025,8 +1026,8 @@ constexpr int64_t partial_floats(int kMT) { return (int64_t)kGemmThreads * 64 * 
 // loop spends no vector ALU work on their addresses (check_offsets bounds
 // every offset below 2^31).
 template <int kMT>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t activation_setup(const GemmArgs &g, int64_t m0,
-                                                                   int lane, uint32_t (&aoff)[4 * kMT]) {
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t activation_setup(
+    const GemmArgs &g, int64_t m0, int lane, uint32_t (&aoff)[4 * kMT]) {
   const int64_t mb = (m0 < g.M) ? m0 : g.M - 1;
   const char *abase = reinterpret_cast<const char *>(g.a + mb * g.lda + kStep * g.k0);
   // Rows available to this wave from mb (at least 1, at most 32 kMT).
@@ -1202,8 +1203,8 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs &g, const floatx16
 // of the tile loop and spilled 57 registers; store_tile_lds now keeps them
 // in place.)
 template <int kMT>
-__device__ __forceinline__ void epilogue(const GemmArgs &g, const floatx16 (&acc)[kMT][4], u32x4 *lds,
-                                         int64_t m0, int64_t o0, int lane) {
+__device__ __forceinline__ void epilogue(const GemmArgs &g, const floatx16 (&acc)[kMT][4],
+                                         u32x4 *lds, int64_t m0, int64_t o0, int lane) {
   if (((reinterpret_cast<uintptr_t>(g.out) & 15) == 0) && ((g.ldo & 7) == 0))
     store_tile_lds<kMT>(g, acc, lds, m0, o0, lane);
   else
@@ -1241,7 +1242,8 @@ __device__ __forceinline__ void fwd_tile(const GroupedArgs &ga, int tile, GemmAr
 // splits), each over split_steps reduction steps from step slice *
 // split_steps, whose fp32 partials go to the workspace.
 template <int kMT, class Producer>
-__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_fwd_kernel(const GroupedArgs ga) {
+__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1)
+    nf4_gemm_fwd_kernel(const GroupedArgs ga) {
   __shared__ GemmLds<kMT> lds;
   const int T = ga.base.tiles_m * ga.tiles_o;
   const int U = ga.full_tiles + (T - ga.full_tiles) * ga.splits;
@@ -1276,7 +1278,8 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_fwd_k
     prod.init(g, o0, (uint32_t)(uintptr_t)(lds_void_t *)&lds.b[0][0]);
     floatx16 acc[kMT][4];
     zero_acc<kMT>(acc);
-    gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0], lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
+    gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0],
+                             lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
     if (slice < 0) {
       epilogue<kMT>(g, acc, &lds.a[wave][0][0], m0, o0, lane);
     } else {
@@ -1446,7 +1449,8 @@ __device__ __forceinline__ void store_swiglu(const GemmArgs &g, const floatx16 (
 // 2-3), so each tile does the MFMA work of a 128-column tile and writes half
 // the output bytes.  grp[0] is the gate weight, grp[1] the up weight.
 template <int kMT, class Producer>
-__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_swiglu_kernel(const GroupedArgs ga) {
+__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1)
+    nf4_gemm_swiglu_kernel(const GroupedArgs ga) {
   __shared__ GemmLds<kMT> lds;
   const int T = ga.base.tiles_m * ga.tiles_o;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1476,7 +1480,8 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_swigl
     prod.init(gp, wave < 2 ? c0 : c0 - 64, (uint32_t)(uintptr_t)(lds_void_t *)&lds.b[0][0]);
     floatx16 acc[kMT][4];
     zero_acc<kMT>(acc);
-    gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0], lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
+    gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0],
+                             lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
     store_swiglu<kMT>(g, acc, m0, c0, jl, grp);
   }
 }
@@ -1493,7 +1498,8 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_swigl
 // launch without a split runs the kSplit = false instantiation, which keeps
 // none of the slice bookkeeping.
 template <int kMT, class Producer, bool kSplit>
-__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_dgrad_kernel(const GroupedArgs ga) {
+__global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1)
+    nf4_gemm_dgrad_kernel(const GroupedArgs ga) {
   __shared__ GemmLds<kMT> lds;
   const int T = ga.base.tiles_m * ga.base.tiles_o;
   const int U = kSplit ? ga.full_tiles + (T - ga.full_tiles) * ga.splits : T;
@@ -1538,8 +1544,8 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_dgrad
         const __amdgpu_buffer_rsrc_t arsrc = activation_setup<kMT>(g, m0, lane, aoff);
         Producer prod;
         prod.init(g, o0, (uint32_t)(uintptr_t)(lds_void_t *)&lds.b[0][0]);
-        gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0],
-                            lds.b[0], lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
+        gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0],
+                                 lds.b[1], arsrc, aoff, (int)(g.R / kStep), jl, grp);
       }
       epilogue<kMT>(g, acc, &lds.a[wave][0][0], m0, o0, lane);
     } else {
@@ -1566,8 +1572,8 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_dgrad
           const __amdgpu_buffer_rsrc_t arsrc = activation_setup<kMT>(g, m0, lane, aoff);
           Producer prod;
           prod.init(g, o0, (uint32_t)(uintptr_t)(lds_void_t *)&lds.b[0][0]);
-          gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0],
-                              lds.b[0], lds.b[1], arsrc, aoff, hi - lo, jl, grp);
+          gemm_main<kMT, Producer>(g, prod, acc, &lds.a[wave][0][0], &lds.a[wave][1][0], lds.b[0],
+                                   lds.b[1], arsrc, aoff, hi - lo, jl, grp);
         }
         gbase += steps;
       }
@@ -1587,7 +1593,10 @@ __global__ void __launch_bounds__(kGemmThreads, kMT == 1 ? 2 : 1) nf4_gemm_dgrad
   }
 }
 
-// Workgroups of a kMT launch that the chip runs at once.
+// Workgroups of a kMT launch that the chip runs at once.  Every GEMM launch is
+// persistent: a grid of at most that many workgroups, each looping over tiles
+// b, b + grid, ..., so that a tile's output stores drain while the same
+// workgroup's next tile starts loading.
 inline int64_t launch_slots(int kmt) { return (kmt == 1 ? 2 : 1) * (int64_t)cu_slots(); }
 
 inline uint32_t launch_grid(int kmt, int64_t units) {

@@ -188,7 +188,8 @@ __device__ __forceinline__ bool sk_vec_ok(const uint16_t *out, int64_t ldo) {
 // k-group take 32 gate rows, odd ones the same 32 up rows, and hidden is
 // elementwise between their partial tiles.
 template <int TR, int WN, int WK, bool kSwiglu, bool kDQ>
-__global__ void __launch_bounds__(64 * WN * WK, TR <= 64 ? 4 : 2) nf4_skinny_kernel(const SkinnyArgs a) {
+__global__ void __launch_bounds__(64 * WN * WK, TR <= 64 ? 4 : 2)
+    nf4_skinny_kernel(const SkinnyArgs a) {
   static_assert(!kSwiglu || WN % 2 == 0, "gate and up rows in pairs of waves");
   constexpr int TM = TR < 32 ? 1 : TR / 32;
   constexpr int kCols = 32 * (kSwiglu ? WN / 2 : WN);  // output columns of the workgroup
