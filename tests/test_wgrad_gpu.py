@@ -64,7 +64,7 @@ def test_wgrad_exact_on_integers():
 
 
 # Launches whose rounds are all full take the XCD-block tile order (each
-# XCD's workgroups cover 4 x 8 tiles per round): 256 and 512 tiles, with
+# XCD's workgroups cover 8 x 8 128-row tiles per round): 512 and 1024 tiles, with
 # ragged tokens, a ragged last tile row and accumulate.  Small integers make
 # every element exact, so this pins the order's tile coordinates bit for bit.
 @pytest.mark.parametrize("m,n,k,acc", [(64, 4096, 4096, False), (100, 8128, 2048, True),
