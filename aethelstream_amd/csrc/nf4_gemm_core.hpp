@@ -1642,48 +1642,48 @@ struct LaunchPlan {
 };
 
 // Time of a 64-deep step of a round in which `busy` of the `slots` workgroups
-// that the chip runs at once have a tile, in us: measured at K = 1024 to 28672
-// (weights from HBM, forward and input gradient alike) on a nearly idle chip,
-// at half the slots and at all of them, straight lines between.  Fewer
-// workgroups share the caches, the memory and the power: 172 tiles of 512 rows
-// on 256 CUs take 1.28 us a step where 256 take 1.66, and a plan that
-// charged the full step preferred 258 tiles of 384 rows for them (777 tokens,
-// 11008 x 4096: 99 us against 84).  With kMT = 1 the second half of the slots
-// is a second workgroup on each CU: one step more is then a step of two.
+// that the chip runs at once have a tile, in us: constant up to half the slots,
+// a straight line from there to all of them (fitted with the constants of
+// plan_launch).  Fewer workgroups share the caches, the memory and the power:
+// 172 tiles of 512 rows on 256 CUs take 1.3 us a step where 256 take 1.65, and
+// a plan that charged the full step preferred 258 tiles of 384 rows for them
+// (777 tokens, 11008 x 4096: 98 us against 82).  With kMT = 1 the second half
+// of the slots is a second workgroup on each CU: one tile more is then a step
+// of two.
 inline double step_us(int kmt, int64_t busy, int64_t slots) {
-  constexpr double kIdle[5] = {0, 0.45, 0.70, 0.88, 0.98};
-  constexpr double kHalf[5] = {0, 0.78, 0.80, 1.04, 1.18};
-  constexpr double kPast[5] = {0, 0.95, 0.80, 1.04, 1.18};  // just past half
-  constexpr double kFull[5] = {0, 1.30, 1.02, 1.32, 1.66};
+  constexpr double kHalf[5] = {0, 0.78, 0.87, 1.00, 1.26};
+  constexpr double kFull[5] = {0, 1.25, 1.01, 1.34, 1.65};
   const double f = 2.0 * (double)busy / (double)slots;
-  return f <= 1.0 ? kIdle[kmt] + (kHalf[kmt] - kIdle[kmt]) * f
-                  : kPast[kmt] + (kFull[kmt] - kPast[kmt]) * (f - 1.0);
+  if (f <= 1.0) return kmt == 1 ? 0.34 + (kHalf[1] - 0.34) * f : kHalf[kmt];
+  const double past = kmt == 1 ? 1.12 : kHalf[kmt];
+  return past + (kFull[kmt] - past) * (f - 1.0);
 }
 
 // The row-block size, with or without a split of its last round, whose rounds
 // take the least time.  Larger tiles cost less per row (the dequantization and
 // the weight fragment reads serve more of them), smaller ones leave fewer rows
-// and CUs idle.  A round adds about 5 us (prologue and output burst); a split
-// round 8 to 12.5 for that, short slices and the second launch, and its
-// partials (0.25 us per MiB written and read); 512-row tiles get 2 %, about
-// what the sums err by over several rounds.  Over 1010 shapes (128 to 8192
-// rows, 4 to 256 output tiles, K = 512 to 28672, both directions, widths that
-// take 16-byte stores and not) the choice takes 0.6 % more time than the best
-// of the eight on average, and nowhere more than 2 % over 512-row tiles.
-// Against those for everything, same box: forward 28672 x 8192 at 256 tokens
-// 178 -> 143 us, 384 tokens 195 -> 180 us; 8192 x 8192 at 256 tokens 66 -> 49
-// us; input gradient of 8192 x 8192 at 128 tokens 81 -> 39 us.
+// and CUs idle.  A round adds its prologue and output burst (kRoundUs); a split
+// round its short slices and second launch instead (kSplitUs) and its partials
+// (kPartialUsPerMiB, written and read).  The constants are fitted to the times
+// of all the choices at 5887 random shapes (16 to 8192 rows, 1 to 3 weights of
+// 512 to 28672 outputs of any width, K = 1024 to 28672; forward, SwiGLU and
+// input gradient): the choice takes 0.37 % more time than the best of the eight
+// on average (0.24 % without a workspace) and 0.74 of the time of 512-row
+// tiles; it is 5 % slower than those at 0.2 % of the shapes.
+// Against those, same box: forward 28672 x 8192 at 256 tokens 178 -> 117 us,
+// 384 tokens 188 -> 157 us; 8192 x 8192 at 256 tokens 75 -> 48 us; input
+// gradient of 8192 x 8192 at 128 tokens 78 -> 35 us.
 // Only splits whose partials fit in ws_bytes of workspace are candidates; the
 // others' costs do not depend on it, so a call with the plan_bytes of its
 // sizes, or more, runs the plan they stand for.
 inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int unroll,
                               int64_t ws_bytes) {
-  constexpr double kRoundUs = 5.0, kPartialUsPerMiB = 0.25;
-  constexpr double kSplitUs[5] = {0, 8.0, 10.5, 9.0, 12.5};
+  constexpr double kRoundUs[5] = {0, 5.0, 5.4, 7.4, 11.0};
+  constexpr double kSplitUs[5] = {0, 7.0, 9.4, 11.2, 16.0};
+  constexpr double kPartialUsPerMiB = 0.20;
   LaunchPlan best{};
   double best_us = 0;
   auto offer = [&](const LaunchPlan &p, double us) {
-    if (p.kmt == 4) us *= 0.98;
     if (best.kmt == 0 || us < best_us) {
       best = p;
       best_us = us;
@@ -1698,24 +1698,21 @@ inline LaunchPlan plan_launch(int64_t m, int64_t tiles_o, int64_t nsteps, int un
     int64_t T;
     if (__builtin_mul_overflow(p.tiles_m, tiles_o, &T) || T > kMaxTiles) continue;
     const int64_t slots = launch_slots(kmt), r = T % slots;
-    const double whole =
-        (double)(T / slots) * (step_us(kmt, slots, slots) * nsteps + kRoundUs);
-    double unsplit = whole + (r > 0 ? step_us(kmt, r, slots) * nsteps + kRoundUs : 0.0);
+    auto round_us = [&](int64_t busy) {
+      return step_us(kmt, busy, slots) * nsteps + kRoundUs[kmt];
+    };
+    const double whole = (double)(T / slots) * round_us(slots);
     p.split = split_plan(T, nsteps, unroll, slots);
     if (p.split.tail_tiles > 0) {
       const int64_t tail = p.split.tail_tiles * p.split.splits;
       p.bytes = tail * partial_floats(kmt) * (int64_t)sizeof(float);
-      const double split = whole + step_us(kmt, tail, slots) * p.split.split_steps +
-                           kSplitUs[kmt] + kPartialUsPerMiB * (double)(p.bytes >> 20);
-      if (p.bytes <= ws_bytes) offer(p, split);
-      // After whole rounds the slices are never the slower way: they also
-      // halve the output burst of rows that don't take 16-byte stores (830 x
-      // 36497 over K = 2048: 215 us split, 234 not).
-      if (T > slots && unsplit < split) unsplit = split;
+      if (p.bytes <= ws_bytes)
+        offer(p, whole + step_us(kmt, tail, slots) * p.split.split_steps + kSplitUs[kmt] +
+                     kPartialUsPerMiB * (double)(p.bytes >> 20));
     }
     p.split = SplitPlan{0, 1, 0};
     p.bytes = 0;
-    offer(p, unsplit);
+    offer(p, whole + (r > 0 ? round_us(r) : 0.0));
   }
   return best;
 }

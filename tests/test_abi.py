@@ -186,6 +186,19 @@ def test_plans_count_the_idle_part_of_a_round():
         assert out.value == 0
 
 
+def test_plans_count_the_round_of_each_size():
+    """A round of 512-row tiles costs more beside its steps than a smaller
+    one: 936 x 659 over K = 24320 takes 48 tiles of 256 rows in 5 slices each
+    (57 us as 12 tiles of 512 rows in 19 slices, 51 us so)."""
+    if torch_has_gpu():
+        return
+    lib = _lib.load()
+    out = ctypes.c_int64(-1)
+    ns = (ctypes.c_int64 * 1)(659)
+    assert lib.nf4s_gemm_fwd_workspace_size(ns, 1, 936, 24320, ctypes.byref(out)) == 0
+    assert out.value == 48 * 5 * 256 * 128 * 4
+
+
 def torch_has_gpu():
     import torch
     return torch.cuda.is_available()
