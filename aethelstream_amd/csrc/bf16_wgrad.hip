@@ -514,13 +514,17 @@ __global__ void fill_zero_f32(float *__restrict__ p, int64_t n) {
 // tiles, two workgroups a CU).  Two workgroups hide one's stores and first
 // loads behind the other's products, and half tiles leave less of a last round
 // idle; but each x fragment feeds half the products.  The costs below are in
-// full rounds of 256-row tiles, fitted to 852 shapes (16 to 8192 tokens, 512 to
-// 56000 rows, 1024 to 16384 columns, a tenth of a round to 27): the choice
-// takes 0.4 % more time than the better of the two on average.
+// full rounds of 256-row tiles, fitted to 1214 calls (16 to 8192 tokens, 512 to
+// 56000 rows, 1024 to 16384 columns, stored and accumulated, a tenth of a round
+// to 27): the choice takes 0.3 % more time than the better of the two on
+// average.
 // One round of 128-row tiles (two a CU) takes 0.78 at 256 tokens and 0.055 more
 // with each doubling, in a row of rounds 0.84 and 0.045 (8192 x 8192: 256
 // tokens 57 us against 76, 1000 tokens 130 against 146, 2048 tokens 234 against
-// 242, 4096 tokens 432 against 421, 8192 tokens 850 against 808).  Once the
+// 242, 4096 tokens 432 against 421, 8192 tokens 850 against 808); past the third
+// the workgroups of a patch run out of step and share less, 0.06 a round
+// (accumulated 35816 x 8840 over 2282 tokens, 19 rounds: 1853 us against 1504;
+// stored 27928 x 9144 over 2219, 15 rounds: 1078 against 1003).  Once the
 // operands come near the Infinity Cache's 256 MB, dy comes from memory in rows
 // of 256 bytes: up to 1.3 times that (27176 x 2528 over 8000 tokens 1138 us
 // against 977, 39848 x 7184 over 6783 tokens 1.45 times).
@@ -548,7 +552,9 @@ static int wg_tile_mt(const int64_t *ns, int32_t count, int64_t m, int64_t k, in
   const double two = t2 < 2 * cus ? 0.50 : 0.57;
   const double part2 = f2 == 0.0 ? 0.0 : (f2 <= 0.5 ? 0.40 + 0.4 * f2 : two + 0.5 * f2);
   const double part4 = f4 == 0.0 ? 0.0 : (f4 <= 0.5 ? 0.62 + 0.16 * f4 : 0.40 + 0.6 * f4);
-  const double cost2 = far * ((0.84 + 0.045 * doublings) * (double)(t2 / (2 * cus)) +
+  const double whole = (double)(t2 / (2 * cus));
+  const double late = whole > 3.0 ? 0.06 * (whole - 3.0) : 0.0;
+  const double cost2 = far * ((0.84 + 0.045 * doublings) * whole + late +
                               (0.78 + 0.055 * doublings) * part2);
   const double cost4 = (double)(t4 / cus) + part4;
   return cost2 < cost4 ? 2 : 4;
